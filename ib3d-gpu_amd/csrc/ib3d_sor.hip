@@ -20,6 +20,9 @@
 //             pair also supplies the x neighbours); colour rows have even
 //             length so every pair is an aligned vector access, and the
 //             coefficients are hoisted out of the z loop.
+//   k_sor_block  (ib3d_sor_block.h) two whole sweeps of a block of cells in one
+//             launch, out of registers and LDS: grids up to 1.5 M cells (FP64)
+//             and 2 M (FP32) in modes 0 to 3.
 //   k_sor     one cell per thread: the smoother on the coarse multigrid
 //             levels, where a z-marching thread would have too few peers.
 //   k_resid_pz  FP64 residual b/dt - A p over both colours (optionally of
@@ -214,6 +217,8 @@ __host__ __device__ __forceinline__ bool interior_cell(const SorGeom &g, int ii,
 // rounding only perturbs the inner iterate; the FP64 outer residual decides).
 __device__ __forceinline__ double sor_div(double a, double b) { return a / b; }
 __device__ __forceinline__ float sor_div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+
+#include "ib3d_sor_block.h"
 
 // One colour half-sweep, one cell per thread.
 // FIRST: the unknown starts from zero (own old value and, for the red
@@ -1421,8 +1426,10 @@ int sor_float_tables(Ctx &c) {
 void gmres_release();
 void mg_release();
 void cycle_graph_release();
+static void block_release();
 void sor_release_tables() {
     cycle_graph_release();
+    block_release();
     mg_release();
     gmres_release();
     if (g_axf) { (void)hipFree(g_axf); (void)hipFree(g_ayf); (void)hipFree(g_azf); }
@@ -1556,11 +1563,240 @@ static void sweep32(Ctx &c, double omega, bool first, bool apply, const double *
     }
 }
 
+// ---------------------------------------------------- temporally blocked sweeps
+// Second buffers of k_sor_block's src -> dst launches, the slots of its TRACK
+// form, and the pinned mirror and events through which a solve reads one batch
+// of results while the next runs.
+static double *g_pc2 = nullptr;          // 2*NC doubles (both colours)
+static float *g_e2 = nullptr;            // 2*NC floats, zero where never written
+static int64_t g_pc2_nc = 0, g_e2_nc = 0;
+static constexpr int kTrackBatch = 64;   // launches per batch of the reference rule
+static constexpr int kTrackSlots = 2 * kBlockSub;   // per launch of two sweeps
+static constexpr int64_t kRegion = (int64_t)kTrackBatch * kTrackSlots;
+static double *g_track = nullptr;        // two regions of kRegion doubles
+static double *g_mirror = nullptr;       // pinned, the same
+static hipEvent_t g_batch_ev[2] = {};
+
+static void block_release() {
+    if (g_pc2) (void)hipFree(g_pc2);
+    if (g_e2) (void)hipFree(g_e2);
+    if (g_track) (void)hipFree(g_track);
+    if (g_mirror) (void)hipHostFree(g_mirror);
+    for (auto &e : g_batch_ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    g_pc2 = g_track = g_mirror = nullptr;
+    g_e2 = nullptr;
+    g_pc2_nc = g_e2_nc = 0;
+}
+
+static int batch_mirror() {
+    for (auto &e : g_batch_ev)
+        if (!e) IB3D_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!g_mirror) IB3D_CHECK(hipHostMalloc((void **)&g_mirror, 2 * kRegion * sizeof(double), hipHostMallocDefault));
+    return 0;
+}
+
+// the second FP64 buffer, a copy of pc (the launches write interior cells
+// only; walls and padding have to agree)
+static int second_pc(Ctx &c) {
+    if (g_pc2_nc != c.NC) {
+        if (g_pc2) (void)hipFree(g_pc2);
+        g_pc2 = nullptr;
+        g_pc2_nc = 0;
+        IB3D_CHECK(hipMalloc(&g_pc2, 2 * c.NC * sizeof(double)));
+        g_pc2_nc = c.NC;
+    }
+    for (int col = 0; col < 2; col++)
+        IB3D_CHECK(hipMemcpyAsync(g_pc2 + col * c.NC, c.pc[col], c.NC * sizeof(double), hipMemcpyDeviceToDevice,
+                                  c.stream));
+    return 0;
+}
+
+// the second FP32 buffer: every interior cell is written before it is read,
+// the rest stays 0
+static int second_e(Ctx &c) {
+    if (g_e2_nc == c.NC) return 0;
+    if (g_e2) (void)hipFree(g_e2);
+    g_e2 = nullptr;
+    g_e2_nc = 0;
+    IB3D_CHECK(hipMalloc(&g_e2, 2 * c.NC * sizeof(float)));
+    IB3D_CHECK(dzero(g_e2, 2 * c.NC * sizeof(float)));
+    g_e2_nc = c.NC;
+    return 0;
+}
+
+// Block shapes by grid size.  A CU works on one block of 24 x 16 x 8 (98 KB of
+// LDS in FP64) or a few small ones, so a small grid wants blocks small enough
+// to reach every CU, and a large one blocks with little halo.  us per FP64
+// sweep (TRACK) on 8x8x4 | 8x8x8 | 24x16x8 blocks and with half-sweep launches:
+// 18k cells 3.5 | 4.3 | 6.5 | 14.9, 49k 4.1 | 4.4 | 6.5 | 17.6, 147k
+// 6.3 | 6.0 | 6.9 | 17.8, 301k 10.0 | 7.7 | 7.5 | 18.7, 524k 14.9 | 11.2 | 8.2 |
+// 16.5, 1.47M - | 22.3 | 15.1 | 20.1, 1.70M - | 27.5 | 20.9 | 21.3.  FP32 on
+// 24x8x8: 3.0-3.3 up to 147k, 4.8 at 524k, 8.3 at 1.47M, 9.9 at 1.70M (half-
+// sweeps 11.6-15.5).
+enum { kBlockNone = 0, kBlock884, kBlock888, kBlock24168, kBlock2488 };
+static int block_shape(const Ctx &c, bool fp64) {
+    const int64_t cells = c.nx * c.ny * c.nz;
+    if (c.NC >= (int64_t)1 << 28) return kBlockNone;   // 32-bit byte offsets into a colour array
+    if (!fp64) return cells <= 2000000 ? kBlock2488 : kBlockNone;
+    if (cells > 1500000) return kBlockNone;
+    // block_div's denominators: every diagonal in [-2^64, -2^-64], as any grid
+    // of non-extreme spacings gives (the sums of the axes' extremes bound them)
+    double lo = 0.0, hi = 0.0;
+    const std::vector<double> *A[3] = {&c.hAcx, &c.hAcy, &c.hAcz};
+    const int64_t n[3] = {c.nx, c.ny, c.nz};
+    for (int a = 0; a < 3; a++) {
+        double mn = HUGE_VAL, mx = -HUGE_VAL;
+        for (int64_t i = 0; i < n[a]; i++) {
+            const double v = (*A[a])[i + n[a]];
+            if (!std::isfinite(v)) return kBlockNone;
+            mn = std::min(mn, v);
+            mx = std::max(mx, v);
+        }
+        lo += mn;
+        hi += mx;
+    }
+    if (!(hi <= -0x1p-64 && lo >= -0x1p64)) return kBlockNone;
+    return cells <= 65536 ? kBlock884 : cells <= 262144 ? kBlock888 : kBlock24168;
+}
+
+template <typename T, int M, int OX, int OY, int OZ, bool FIRST, bool TRACK, bool APPLY>
+static void launch_block(Ctx &c, const T *s0, const T *s1, T *d0, T *d1, const T *r0, const T *r1, const T *ax,
+                         const T *ay, const T *az, T omega, T omm, const double *gate, double thr,
+                         const double *prev, double *slot, double *acc0, double *acc1) {
+    const int nbx = (int)((c.nx + OX - 1) / OX), nby = (int)((c.ny + OY - 1) / OY), nbz = (int)((c.nz + OZ - 1) / OZ);
+    hipLaunchKernelGGL((k_sor_block<T, M, OX, OY, OZ, FIRST, TRACK, APPLY>), dim3((unsigned)(nbx * nby * nbz)),
+                       dim3((BlockShape<M, OX, OY, OZ>::NT)), 0, c.stream, s0, s1, d0, d1, r0, r1, ax, ay, az,
+                       geom(c), nbx, nby, omega, omm, gate, thr, prev, slot, acc0, acc1);
+}
+
+// M (1 or 2) FP64 sweeps between pc (buffer 0) and g_pc2 (buffer 1), from
+// buffer `from`; TRACK (M = 2) when slot is given
+static void block64(Ctx &c, int shape, int M, int from, double omega, const double *gate, double thr,
+                    const double *prev = nullptr, double *slot = nullptr) {
+    double *b[2][2] = {{c.pc[0], c.pc[1]}, {g_pc2, g_pc2 + c.NC}};
+    double **s = b[from], **d = b[1 - from];
+    const double omm = 1.0 - omega;
+#define IB3D_BLOCK(MM, TR, X, Y, Z)                                                                                 \
+    launch_block<double, MM, X, Y, Z, false, TR, false>(c, s[0], s[1], d[0], d[1], c.bdt[0], c.bdt[1], c.ax, c.ay,   \
+                                                        c.az, omega, omm, gate, thr, prev, slot, nullptr, nullptr)
+#define IB3D_SHAPES(MM, TR)                                                                                         \
+    do {                                                                                                            \
+        if (shape == kBlock884) IB3D_BLOCK(MM, TR, 8, 8, 4);                                                        \
+        else if (shape == kBlock888) IB3D_BLOCK(MM, TR, 8, 8, 8);                                                   \
+        else IB3D_BLOCK(MM, TR, 24, 16, 8);                                                                         \
+    } while (0)
+    if (slot) IB3D_SHAPES(2, true);
+    else if (M == 2) IB3D_SHAPES(2, false);
+    else IB3D_SHAPES(1, false);
+#undef IB3D_SHAPES
+#undef IB3D_BLOCK
+}
+
+// M FP32 sweeps of the right-hand side r (both colours), src -> dst; first:
+// from zero; acc0: first add src to the FP64 unknown
+static void block32(Ctx &c, int M, const float *src, float *dst, const float *r, double omega, bool first,
+                    const double *gate, double *acc0 = nullptr, double *acc1 = nullptr) {
+    const float om = (float)omega, omm = (float)(1.0 - omega);
+    const int64_t NC = c.NC;
+#define IB3D_BLOCK(MM, F, A)                                                                                        \
+    launch_block<float, MM, 24, 8, 8, F, false, A>(c, src, src + NC, dst, dst + NC, r, r + NC, g_axf, g_ayf, g_azf,  \
+                                                   om, omm, gate, 0.5, nullptr, nullptr, acc0, acc1)
+    if (M == 2) {
+        if (first && acc0) IB3D_BLOCK(2, true, true);
+        else if (first) IB3D_BLOCK(2, true, false);
+        else IB3D_BLOCK(2, false, false);
+    } else {
+        if (first && acc0) IB3D_BLOCK(1, true, true);
+        else if (first) IB3D_BLOCK(1, true, false);
+        else IB3D_BLOCK(1, false, false);
+    }
+#undef IB3D_BLOCK
+}
+
+// n >= 2 sweeps as an even number of launches, so that a -> b -> a ends where
+// it began: two sweeps each, then single ones.  calls f(sweeps, launch index).
+template <typename F> static void even_launches(int n, F f) {
+    int two = n / 2, one = n % 2;
+    if ((two + one) % 2) {
+        two--;
+        one += 2;
+    }
+    for (int q = 0; q < two + one; q++) f(q < two ? 2 : 1, q);
+}
+
+// The reference rule on blocks: launches of two sweeps, queued in batches one
+// ahead of the batch the host reads, so the GPU never waits for the host.  The
+// launch in which a sweep falls below epsi stops those after it; if that was
+// its first sweep, it is repeated from its source with one.  Batches are large
+// until the previous solve's count is near, small after: a launch queued after
+// convergence still costs about 3 us.
+static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, double *derr2) {
+    const double omega = 1.99;
+    if (batch_mirror() || second_pc(c)) return -1;
+    if (!g_track) IB3D_CHECK(hipMalloc(&g_track, 2 * kRegion * sizeof(double)));
+    // the sweep count past which the plain loop below gives up: the first sum
+    // of its batches above the cap
+    int64_t cap = 0, step = std::max(1, c.batch);
+    for (; cap <= c.max_sweeps && step < 256; step = std::min<int64_t>(step * 2, 256)) cap += step;
+    if (cap <= c.max_sweeps) cap += ((c.max_sweeps - cap) / step + 1) * step;
+    int64_t queued = 0, seen = 0;   // launches
+    int size[2] = {0, 0};
+    const double *prev = nullptr;
+    for (int batch = 0;; batch++) {
+        const int reg = batch & 1;
+        const int64_t left = c.last_ref / 2 - queued;
+        const int n = left >= 96 ? kTrackBatch : left >= 48 ? 32 : 16;
+        double *region = g_track + reg * kRegion;
+        IB3D_CHECK(hipMemsetAsync(region, 0, n * kTrackSlots * sizeof(double), c.stream));
+        for (int q = 0; q < n; q++) {
+            double *slot = region + q * kTrackSlots;
+            block64(c, shape, 2, (int)((queued + q) & 1), omega, nullptr, epsi, prev, slot);
+            prev = slot;
+        }
+        IB3D_CHECK(hipGetLastError());
+        IB3D_CHECK(hipMemcpyAsync(g_mirror + reg * kRegion, region, n * kTrackSlots * sizeof(double),
+                                  hipMemcpyDeviceToHost, c.stream));
+        IB3D_CHECK(hipEventRecord(g_batch_ev[reg], c.stream));
+        queued += n;
+        size[reg] = n;
+        if (batch == 0) continue;
+        const int old = 1 - reg;
+        IB3D_CHECK(hipEventSynchronize(g_batch_ev[old]));
+        for (int q = 0; q < size[old]; q++, seen++) {
+            for (int w = 0; w < 2; w++) {
+                const double *h = g_mirror + old * kRegion + q * kTrackSlots + w * kBlockSub;
+                const double v = *std::max_element(h, h + kBlockSub);
+                const int64_t it = 2 * seen + w + 1;
+                if (it > cap) {
+                    set_error("REDBLACKSOR: no convergence within the sweep cap");
+                    return -1;
+                }
+                if (v >= epsi) continue;  // the reference loops while derr2 >= epsi
+                const int from = (int)(seen & 1);
+                if (w == 0) block64(c, shape, 1, from, omega, nullptr, 0.0);
+                if (from == 0)   // the result is in the second buffer
+                    for (int col = 0; col < 2; col++)
+                        IB3D_CHECK(hipMemcpyAsync(c.pc[col], g_pc2 + col * c.NC, c.NC * sizeof(double),
+                                                  hipMemcpyDeviceToDevice, c.stream));
+                IB3D_CHECK(hipGetLastError());
+                *isum = it;
+                *derr2 = v;
+                c.last_sweeps = c.last_ref = it;
+                return 0;
+            }
+        }
+    }
+}
+
 // subPcorVcor.f90:148-212 with the reference stopping rule.  Iterations are
 // queued in batches; each kernel first checks whether the previous
 // iteration already converged, so the result (and the count) equals the
 // one-iteration-at-a-time loop while the host synchronises once per batch.
 int redblack_sor_reference(Ctx &c, double epsi, int64_t *isum, double *derr2) {
+    if (const int shape = block_shape(c, true)) return reference_blocks(c, shape, epsi, isum, derr2);
     const double omega = 1.99;
     int64_t done = 0;
     int batch = std::max(1, c.batch);
@@ -1637,6 +1873,7 @@ static int sor_l2(Ctx &c, bool mixed, double bn, int64_t *sweeps, int64_t *outer
     if (ensure_partial(nblocks(2 * c.NC, kSorBlock))) return -1;
     const int64_t max_outer = std::max<int64_t>(1, c.max_sweeps / c.check);
     if (ensure_slots(2 * (max_outer + 2))) return -1;
+    if (batch_mirror()) return -1;
     double *relv = c.slots, *conv = c.slots + c.n_slots / 2;
     hipLaunchKernelGGL(k_clear_dead, dim3(nblocks(2 * c.NC, kSorBlock)), dim3(kSorBlock), 0, c.stream, c.pc[0],
                        c.pc[1], c.e32[0], c.e32[1], c.bdt[0], c.bdt[1], c.NC);
@@ -1649,60 +1886,83 @@ static int sor_l2(Ctx &c, bool mixed, double bn, int64_t *sweeps, int64_t *outer
         IB3D_CHECK(hipGetLastError());
         if (cnn_before_solve(c, c.scalars + 16, c.scalars + 18, resid_rel)) return -1;
     }
+    // temporally blocked launches where they pay and the sweeps of an outer
+    // iteration can end in the buffer they began in
+    const int shape = c.check >= 2 ? block_shape(c, !mixed) : kBlockNone;
+    if (shape && (mixed ? second_e(c) : second_pc(c))) return -1;
     residual_async(c, false, mixed, bn, relv, conv, nullptr);
     int64_t o = 0;     // last queued outer iteration
     int64_t seen = 0;  // first index not yet inspected on the host
-    // the previous solve's count predicts this one's (warm starts, slowly
-    // varying flow): queue a little less than that first, then grow
-    int batch = (int)std::min<int64_t>(64, std::max<int64_t>(4, c.last_outer - 2));
-    std::vector<double> hr, hc;
-    for (;;) {
+    auto queue = [&](int batch) {
         for (int q = 0; q < batch && o < max_outer; q++) {
             o++;
             const double *gate = conv + (o - 1);
-            for (int s = 0; s < c.check; s++) {
-                if (mixed)
-                    sweep32(c, c.omega, s == 0, s == 0 && o > 1, gate, 0.5);
-                else
-                    sweep64(c, c.omega, false, nullptr, gate, 0.5);
+            if (shape && mixed) {
+                even_launches(c.check, [&](int m, int l) {
+                    const bool apply = l == 0 && o > 1;
+                    block32(c, m, l % 2 ? g_e2 : c.e32[0], l % 2 ? c.e32[0] : g_e2, c.r32[0], c.omega, l == 0, gate,
+                            apply ? c.pc[0] : nullptr, apply ? c.pc[1] : nullptr);
+                });
+            } else if (shape) {
+                even_launches(c.check, [&](int m, int l) { block64(c, shape, m, l % 2, c.omega, gate, 0.5); });
+            } else {
+                for (int s = 0; s < c.check; s++) {
+                    if (mixed)
+                        sweep32(c, c.omega, s == 0, s == 0 && o > 1, gate, 0.5);
+                    else
+                        sweep64(c, c.omega, false, nullptr, gate, 0.5);
+                }
             }
             residual_async(c, mixed, mixed, bn, relv + o, conv + o, gate);
         }
-        IB3D_CHECK(hipGetLastError());
+    };
+    // Batches of outer iterations are queued one ahead of the batch the host
+    // reads (through the pinned mirror), so the GPU never waits for the host.
+    // The previous solve's count predicts this one's (warm starts, slowly
+    // varying flow): a little less than that first, then a few at a time,
+    // since a launch queued after convergence still costs about 2 us.
+    struct Batch { int64_t from, to; };
+    Batch pending[2];
+    static constexpr int64_t kMost = kRegion / 2;   // entries of a region: residuals and flags
+    auto submit = [&](int reg) {
         const int64_t n = o - seen + 1;
-        hr.resize(n);
-        hc.resize(n);
-        IB3D_CHECK(hipMemcpyAsync(hr.data(), relv + seen, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-        IB3D_CHECK(hipMemcpyAsync(hc.data(), conv + seen, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-        IB3D_CHECK(hipStreamSynchronize(c.stream));
-        if (seen == 0) *rel0 = hr[0];
-        for (int64_t q = 0; q < n; q++) {
-            if (!(hr[q] == hr[q]) || !std::isfinite(bn)) {
+        double *m = g_mirror + reg * kRegion;
+        IB3D_CHECK(hipGetLastError());
+        IB3D_CHECK(hipMemcpyAsync(m, relv + seen, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        IB3D_CHECK(hipMemcpyAsync(m + kMost, conv + seen, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        IB3D_CHECK(hipEventRecord(g_batch_ev[reg], c.stream));
+        pending[reg] = {seen, o};
+        seen = o + 1;
+        return 0;
+    };
+    queue((int)std::min<int64_t>(kMost - 1, std::max<int64_t>(4, c.last_outer - 4)));
+    if (submit(0)) return -1;
+    for (int batch = 1;; batch++) {
+        const int reg = batch & 1, old = 1 - reg;
+        const bool more = o < max_outer;
+        if (more) {
+            queue(4);
+            if (submit(reg)) return -1;
+        }
+        IB3D_CHECK(hipEventSynchronize(g_batch_ev[old]));
+        const double *hr = g_mirror + old * kRegion, *hc = hr + kMost;
+        for (int64_t i = pending[old].from; i <= pending[old].to; i++, hr++, hc++) {
+            if (i == 0) *rel0 = *hr;
+            if (!(*hr == *hr) || !std::isfinite(bn)) {
                 set_error("poissonSolver: the residual is not finite");
                 return -1;
             }
-            if (hc[q] < 0.5) {
-                const int64_t oc = seen + q;  // converged after oc outer iterations
-                if (mixed && oc > 0) add_increment(c);
+            // converged after i outer iterations, or at the cap
+            if (*hc < 0.5 || i == max_outer) {
+                if (mixed && i > 0) add_increment(c);
                 IB3D_CHECK(hipGetLastError());
                 if (cnn && cnn_after_solve(c, c.scalars + 16, c.scalars + 18)) return -1;
-                *sweeps = oc * c.check;
-                *outer = oc;
-                *rel = hr[q];
+                *sweeps = i * c.check;
+                *outer = i;
+                *rel = *hr;
                 return 0;
             }
         }
-        if (o >= max_outer) {
-            if (mixed && o > 0) add_increment(c);
-            IB3D_CHECK(hipGetLastError());
-            if (cnn && cnn_after_solve(c, c.scalars + 16, c.scalars + 18)) return -1;
-            *sweeps = o * c.check;
-            *outer = o;
-            *rel = hr[n - 1];
-            return 0;
-        }
-        seen = o + 1;
-        batch = std::min(std::max(batch, 4) * 2, 64);
     }
 }
 
@@ -2781,6 +3041,10 @@ static int gmres_cycle(Ctx &c, int m, int k, const double *gate, double target, 
         float *Z = g_kz + j * stride, *Vj = g_kv + j * stride, *Vn = g_kv + (j + 1) * stride;
         if (c.mode == 4) {
             mg_vcycle(c, Vj, Z, aj);
+        } else if (k >= 2 && block_shape(c, false)) {
+            even_launches(k, [&](int mm, int l) {
+                block32(c, mm, l % 2 ? g_e2 : Z, l % 2 ? Z : g_e2, Vj, c.omega, l == 0, aj);
+            });
         } else {
             for (int sw = 0; sw < k; sw++) {
                 for (int col = 0; col < 2; col++) {
@@ -2899,7 +3163,7 @@ static int cycle_graph(Ctx &c, int m, int k, double *relv, double *conv) {
                           (const void *)c.az, (const void *)c.partial, (const void *)c.scalars, (const void *)relv,
                           (const void *)conv, (const void *)g_axf, (const void *)g_ayf, (const void *)g_azf,
                           (const void *)g_kv, (const void *)g_kz, (const void *)g_kh, (const void *)g_kpart,
-                          (const void *)g_kpart2, (const void *)g_actbits})
+                          (const void *)g_kpart2, (const void *)g_actbits, (const void *)g_e2})
         P(q);
     for (const MgLevel &L : g_mg)
         for (const void *q : {(const void *)L.x, (const void *)L.b, (const void *)L.r, (const void *)L.ax,
@@ -2962,6 +3226,7 @@ static int sor_gmres(Ctx &c, double bn, int64_t *sweeps, int64_t *outer, double 
     if (sor_float_tables(c)) return -1;
     if (gmres_buffers(c, m)) return -1;
     if (c.mode == 4 && mg_setup(c)) return -1;
+    if (c.mode == 3 && k >= 2 && block_shape(c, false) && second_e(c)) return -1;
     if (clear_for_geometry(c, m)) return -1;
     if (ensure_partial(nblocks(2 * c.NC, kSorBlock))) return -1;
     const int64_t max_outer = std::max<int64_t>(1, c.max_sweeps / ((int64_t)m * k));
