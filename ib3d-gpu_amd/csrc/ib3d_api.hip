@@ -117,8 +117,9 @@ static void free_all(Ctx &c) {
     dfree(c.ibList); dfree(c.fluidList); dfree(c.solidList);
     c.cap_lists[0] = c.cap_lists[1] = c.cap_lists[2] = 0;
     c.cap_nel = 0; dfree(c.nel); dfree(c.scell); dfree(c.scontrib);
-    dfree(c.rt_flag); dfree(c.rt_list); dfree(c.rt_count); dfree(c.body);
+    dfree(c.rt_flag); dfree(c.rt_bflag); dfree(c.rt_list); dfree(c.rt_count); dfree(c.body);
     release_plans(c);
+    release_clusters(c);
     if (c.hscal) (void)hipHostFree(c.hscal);
     c.hscal = nullptr;
     for (auto &e : c.ev)
@@ -691,6 +692,7 @@ int ib3d_set_mesh(int64_t n_nodes, const double *xn, const double *yn, const dou
     IB3D_CHECK(h2d(c.ynode, yn, n_nodes * 8));
     IB3D_CHECK(h2d(c.znode, zn, n_nodes * 8));
     IB3D_CHECK(h2d(c.elp, el.data(), el.size() * sizeof(int)));
+    if (set_clusters(c, xn, yn, zn, el.data(), n_elems)) return -1;
     c.ibNodes = n_nodes;
     c.ibElems = n_elems;
     c.norms_ready = c.stress_ready = false;

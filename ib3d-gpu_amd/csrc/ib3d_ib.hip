@@ -83,55 +83,220 @@ __global__ void k_surface_norm(const double *xn, const double *yn, const double 
     cg[n] = (g / len) * inor;
 }
 
-// subSearch.f90:166-247: nearest centroid (first index wins ties of the
-// sqrt distance) and the 8-corner plane test.  sqrt is only evaluated when
-// the squared distance is below the current minimum's: sqrt is monotone, so
-// a larger square can never give a strictly smaller distance.
+// ---- nearest element
+// The reference compares every cell with every element.  Here the elements
+// are grouped into clusters of 64 that lie close together (a Morton order of
+// the mesh, found once per mesh), with the bounding box of each cluster's
+// centroids; a wave of 64 neighbouring cells scans only the clusters that can
+// hold a nearest element of one of them.  The distances are the reference's
+// expressions, and the winner is the reference's: the smallest rounded
+// distance, the first element among equals.
+//
+// Bounded by FP64 arithmetic, 8 operations per pair of cell and element that
+// is left.  With 32768 elements and 9.3 million cells around eight bodies the
+// tagging takes 3.2 ms (all pairs: 89 ms); the retagging of 30 000 cells around
+// a sphere of 20480 elements 0.074 ms (0.44 ms).
+static constexpr int kCluster = 64;
+
+// one wave per cluster: the centroids in cluster order and their box.  A pad
+// sits at infinity (never nearest); NaN centroids are never nearest either and
+// stay out of the box.
+__global__ void __launch_bounds__(256)
+k_clusters(const int *__restrict__ perm, const double *__restrict__ xc, const double *__restrict__ yc,
+           const double *__restrict__ zc, int nc, double *__restrict__ pos, int *__restrict__ id,
+           double *__restrict__ box) {
+    const int c = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    if (c >= nc) return;
+    const int n = nc * kCluster, q = c * kCluster + lane, e = perm[q];
+    const double inf = __builtin_huge_val();
+    const double v[3] = {e < 0 ? inf : xc[e], e < 0 ? inf : yc[e], e < 0 ? inf : zc[e]};
+    id[q] = e < 0 ? 0x7fffffff : e + 1;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        pos[a * n + q] = v[a];
+        double lo = e < 0 ? inf : fmin(v[a], inf), hi = e < 0 ? -inf : fmax(v[a], -inf);
+        for (int off = 32; off > 0; off >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, off, 64));
+            hi = fmax(hi, __shfl_xor(hi, off, 64));
+        }
+        if (lane == 0) {
+            box[a * nc + c] = lo;
+            box[(3 + a) * nc + c] = hi;
+        }
+    }
+}
+
+struct ClusterView {
+    const double *pos, *box;   // centroids [3][64 nc] and boxes [lo xyz, hi xyz][nc]
+    const int *id;             // 1-based element
+    int nc;
+};
+
+// The reference's first nearest element of each lane's point (0: none closer
+// than 1e14), by W waves that hold the same 64 points and share the clusters
+// (part: which of them this wave is; every wave returns the result when W = 1,
+// wave 0 otherwise).  All lanes take part; lo and hi bound the active lanes'
+// points.  Rounding is monotone, so a distance to a box computed with the same
+// operations never exceeds the computed distance to a centroid in it; and an
+// element whose rounded distance equals the best one has its square within a few
+// rounding units of the best's, hence the margin of `slim`.
+template <int W>
+__device__ __forceinline__ int nearest_element(const ClusterView &E, bool active, double px, double py, double pz,
+                                               const double lo[3], const double hi[3], int part) {
+    typedef __attribute__((address_space(4))) double CD;
+    const int lane = threadIdx.x & 63, n = E.nc * kCluster;
+    const double inf = __builtin_huge_val();
+    double minDis = 1e14, slim = inf;
+    int nel = 0;
+    auto take = [&](double dis, int m) {
+        const bool first = dis < minDis || (dis == minDis && m < nel);
+        minDis = first ? dis : minDis;
+        nel = first ? m : nel;
+    };
+    auto scan = [&](int c) {   // c is uniform
+        const double bx = fmax(fmax(E.box[c] - px, px - E.box[3 * E.nc + c]), 0.0);
+        const double by = fmax(fmax(E.box[E.nc + c] - py, py - E.box[4 * E.nc + c]), 0.0);
+        const double bz = fmax(fmax(E.box[2 * E.nc + c] - pz, pz - E.box[5 * E.nc + c]), 0.0);
+        if (!__any(active && !(((by * by) + (bx * bx)) + (bz * bz) > slim))) return;
+        const CD *x = (const CD *)(E.pos + c * kCluster), *y = (const CD *)(E.pos + n + c * kCluster),
+                 *z = (const CD *)(E.pos + 2 * n + c * kCluster);
+        // the next elements are on their way (scalar loads) while these are compared
+        constexpr int G = 4;
+        double ex[G], ey[G], ez[G];
+#pragma unroll
+        for (int t = 0; t < G; t++) {
+            ex[t] = x[t];
+            ey[t] = y[t];
+            ez[t] = z[t];
+        }
+#pragma unroll 2
+        for (int t0 = 0; t0 < kCluster; t0 += G) {
+            const int tn = t0 + G < kCluster ? t0 + G : t0;
+            double nx[G], ny[G], nz[G], s4[G];
+#pragma unroll
+            for (int t = 0; t < G; t++) {
+                nx[t] = x[tn + t];
+                ny[t] = y[tn + t];
+                nz[t] = z[tn + t];
+            }
+#pragma unroll
+            for (int t = 0; t < G; t++) {
+                const double dy = py - ey[t], dx = px - ex[t], dz = pz - ez[t];
+                s4[t] = ((dy * dy) + (dx * dx)) + (dz * dz);
+            }
+            if (fmin(fmin(s4[0], s4[1]), fmin(s4[2], s4[3])) <= slim) {
+#pragma unroll
+                for (int t = 0; t < G; t++)
+                    if (s4[t] <= slim) {
+                        const double dis = sqrt(unhoisted(s4[t]));
+                        if (dis < minDis) slim = s4[t] * (1.0 + 0x1p-49);
+                        take(dis, E.id[c * kCluster + t0 + t]);
+                    }
+            }
+#pragma unroll
+            for (int t = 0; t < G; t++) {
+                ex[t] = nx[t];
+                ey[t] = ny[t];
+                ez[t] = nz[t];
+            }
+        }
+    };
+    // start with the cluster whose farthest point is nearest
+    double best = inf;
+    int bi = 0;
+    for (int c = lane; c < E.nc; c += 64) {
+        double f = 0.0;
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const double d = fmax(E.box[(3 + a) * E.nc + c] - lo[a], hi[a] - E.box[a * E.nc + c]);
+            f += d * d;
+        }
+        if (f < best) {
+            best = f;
+            bi = c;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const double ob = __shfl_xor(best, off, 64);
+        const int oi = __shfl_xor(bi, off, 64);
+        if (ob < best || (ob == best && oi < bi)) {
+            best = ob;
+            bi = oi;
+        }
+    }
+    bi = __builtin_amdgcn_readfirstlane(bi);
+    scan(bi);
+    // then every cluster that is not farther from all the points than their
+    // nearest so far
+    double most = active ? slim : 0.0;
+    for (int off = 32; off > 0; off >>= 1) most = fmax(most, __shfl_xor(most, off, 64));
+    int turn = 0;
+    for (int c0 = 0; c0 < E.nc; c0 += 64) {
+        const int c = c0 + lane;
+        bool keep = false;
+        if (c < E.nc && c != bi) {
+            double d[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+                d[a] = fmax(fmax(E.box[a * E.nc + c] - hi[a], lo[a] - E.box[(3 + a) * E.nc + c]), 0.0);
+            keep = !(((d[1] * d[1]) + (d[0] * d[0])) + (d[2] * d[2]) > most);
+        }
+        for (unsigned long long m = __ballot(keep); m; m &= m - 1)
+            if (W == 1 || turn++ % W == part) scan(c0 + __builtin_ctzll(m));
+    }
+    if (W > 1) {
+        __shared__ double s_dis[W][64];
+        __shared__ int s_nel[W][64];
+        s_dis[part][lane] = minDis;
+        s_nel[part][lane] = nel;
+        __syncthreads();
+        if (part == 0)
+            for (int q = 1; q < W; q++)
+                if (s_nel[q][lane] > 0) take(s_dis[q][lane], s_nel[q][lane]);
+        __syncthreads();   // (the arrays are rewritten by the next call)
+    }
+    return nel;
+}
+
+// bounds of the coordinates f..l of one axis
+__device__ __forceinline__ void axis_bounds(const double *p, int f, int l, double &lo, double &hi) {
+    lo = hi = p[f];
+    for (int q = f + 1; q <= l; q++) {
+        lo = fmin(lo, p[q]);
+        hi = fmax(hi, p[q]);
+    }
+}
+
+// subSearch.f90:166-247: nearest centroid and the 8-corner plane test, a
+// brick of 4 x 4 x 4 cells per W waves.  One wave where the bricks fill the
+// chip (145 000 bricks: 3.2 ms, with four 4.8 ms); four below 8192 of them,
+// where the bricks near a body's centre, which few clusters can be skipped for,
+// are the whole time (46 x 46 x 46 cells and 20480 triangles: 0.37 ms, with one
+// 1.48 ms, all pairs 1.82 ms).
 static constexpr int kTagTile = 256;
+template <int W>
 __global__ void __launch_bounds__(kTagTile)
 k_tagging(int i0, int i1, int j0, int j1, int k0, int k1, int sx, int sy, const double *__restrict__ xp,
           const double *__restrict__ yp, const double *__restrict__ zp, const double *__restrict__ x1,
           const double *__restrict__ y1, const double *__restrict__ z1, const double *__restrict__ xc,
           const double *__restrict__ yc, const double *__restrict__ zc, const double *__restrict__ ca,
-          const double *__restrict__ cb, const double *__restrict__ cg, int ne, int8_t *tag, int *minElem,
+          const double *__restrict__ cb, const double *__restrict__ cg, ClusterView E, int8_t *tag, int *minElem,
           int *err) {
-    __shared__ double sx_[kTagTile], sy_[kTagTile], sz_[kTagTile];
-    const int wi = i1 - i0 + 1, wj = j1 - j0 + 1, wk = k1 - k0 + 1;
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = q < (int64_t)wi * wj * wk;
-    int i = 0, j = 0, k = 0;
-    if (active) {
-        i = i0 + (int)(q % wi);
-        const int64_t r = q / wi;
-        j = j0 + (int)(r % wj);
-        k = k0 + (int)(r / wj);
-    }
+    const int bi = (i1 - i0 + 4) / 4, bj = (j1 - j0 + 4) / 4, bk = (k1 - k0 + 4) / 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kTagTile / 64) + (threadIdx.x >> 6)));
+    const int brick = wave / W, part = wave % W;
+    if (brick >= bi * bj * bk) return;   // (with W = 4, a whole workgroup)
+    const int lane = threadIdx.x & 63;
+    const int ib = i0 + 4 * (brick % bi), jb = j0 + 4 * (brick / bi % bj), kb = k0 + 4 * (brick / bi / bj);
+    const int i = ib + (lane & 3), j = jb + ((lane >> 2) & 3), k = kb + (lane >> 4);
+    const bool active = i <= i1 && j <= j1 && k <= k1;
+    double lo[3], hi[3];
+    axis_bounds(xp, ib, min(ib + 3, i1), lo[0], hi[0]);
+    axis_bounds(yp, jb, min(jb + 3, j1), lo[1], hi[1]);
+    axis_bounds(zp, kb, min(kb + 3, k1), lo[2], hi[2]);
     const double n1x = active ? xp[i] : 0.0, n1y = active ? yp[j] : 0.0, n1z = active ? zp[k] : 0.0;
-    double minDis = 1e14, smin = __builtin_huge_val();
-    int nel = 0;
-    for (int base = 0; base < ne; base += kTagTile) {
-        const int m = base + threadIdx.x;
-        __syncthreads();
-        if (m < ne) {
-            sx_[threadIdx.x] = xc[m];
-            sy_[threadIdx.x] = yc[m];
-            sz_[threadIdx.x] = zc[m];
-        }
-        __syncthreads();
-        const int cnt = min(kTagTile, ne - base);
-        for (int t = 0; t < cnt; t++) {
-            const double dy = n1y - sy_[t], dx = n1x - sx_[t], dz = n1z - sz_[t];
-            const double s = ((dy * dy) + (dx * dx)) + (dz * dz);
-            if (s < smin) {
-                const double dis = sqrt(s);
-                if (dis < minDis) {
-                    minDis = dis;
-                    smin = s;
-                    nel = base + t + 1;
-                }
-            }
-        }
-    }
+    const int nel = nearest_element<W>(E, active, n1x, n1y, n1z, lo, hi, part);
+    if (W > 1 && part != 0) return;
     if (!active) return;
     if (nel < 1) {
         atomicOr(err, 1);
@@ -160,61 +325,36 @@ k_tagging(int i0, int i1, int j0, int j1, int k0, int k1, int sx, int sy, const 
     minElem[c] = nel;
 }
 
-// subSearch.f90:360-363: queue the 6x6x6 block (i1-2..i1+3, ...) around every
-// intercepted cell; each cell enters the list once (the reference tags
-// overlapping blocks repeatedly, always with the same result).  Cells
-// outside the padded index range 1..n+2 are not queued.
-__global__ void __launch_bounds__(1024)
-k_retag_mark(const int *ib, int nb, int nx, int ny, int nz, uint8_t *flag, int *list, int *count) {
-    // one atomicAdd on the list counter per block: a cell's slot = block base
-    // + cells newly queued by lower waves + set ballot bits below its lane
-    __shared__ int s_wave[16];
-    __shared__ int s_base;
+// subSearch.f90:360-363: flag the 6x6x6 block (i1-2..i1+3, ...) around every
+// intercepted cell and queue the 4x4x4 bricks of the grid that hold flagged
+// cells, each once (the reference tags overlapping blocks repeatedly, always
+// with the same result).  Cells outside the padded index range 1..n+2 are not
+// flagged.  A thread flags one row of six cells; the first nine of a block's 36
+// threads queue up to three bricks each: 32 us for 7500 intercepted cells.  (One
+// thread per cell, each asking for its brick, took 280 us: the bricks' few
+// addresses serialise the requests.)
+__global__ void __launch_bounds__(256)
+k_retag_mark(const int *ib, int nb, int nx, int ny, int nz, uint8_t *flag, unsigned int *bflag, int *list,
+             int *count) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    bool add = false;
-    int64_t c = 0;
-    if (q < (int64_t)nb * 216) {
-        const int n = (int)(q / 216), o = (int)(q % 216);
-        const int i = ib[n] - 2 + o % 6, j = ib[nb + n] - 2 + (o / 6) % 6, k = ib[2 * nb + n] - 2 + o / 36;
-        if (i >= 1 && i <= nx + 2 && j >= 1 && j <= ny + 2 && k >= 1 && k <= nz + 2) {
-            c = lin(i, j, k, nx + 2, ny + 2);
-            unsigned int *word = reinterpret_cast<unsigned int *>(flag + (c & ~(int64_t)3));
-            const unsigned int bit = 1u << (8 * (c & 3));
-            // overlapping blocks queue the same cells many times: a relaxed
-            // load that already sees the bit skips the atomic (only the
-            // atomic that sets the bit queues the cell)
-            if (!(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
-                add = !(atomicOr(word, bit) & bit);
-        }
+    if (q >= (int64_t)nb * 36) return;
+    const int n = (int)(q / 36), o = (int)(q % 36);
+    const int i0 = max(ib[n] - 2, 1), i1 = min(ib[n] + 3, nx + 2);
+    const int jm = ib[nb + n], km = ib[2 * nb + n];
+    const int j = jm - 2 + o % 6, k = km - 2 + o / 6;
+    if (j >= 1 && j <= ny + 2 && k >= 1 && k <= nz + 2) {
+        uint8_t *row = flag + lin(0, j, k, nx + 2, ny + 2);
+        for (int i = i0; i <= i1; i++)
+            if (!row[i]) row[i] = 1;
     }
-    const unsigned long long bal = __ballot(add);
-    if (lane == 0) s_wave[wv] = __popcll(bal);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int t = 0; t < (int)(blockDim.x >> 6); t++) {
-            const int v = s_wave[t];
-            s_wave[t] = run;
-            run += v;
-        }
-        s_base = run > 0 ? atomicAdd(count, run) : 0;
-    }
-    __syncthreads();
-    if (add) list[s_base + s_wave[wv] + __popcll(bal & ((1ull << lane) - 1))] = (int)c;
-}
-
-// One step of the first-nearest-element scan: sqrt only when the square is
-// below the current minimum's (sqrt is monotone, so a larger square can
-// never give a strictly smaller distance); ties keep the earlier element.
-__device__ __forceinline__ void nearest_update(double s, int elem1, double &smin, double &minDis, int &nel) {
-    if (s < smin) {
-        const double dis = sqrt(unhoisted(s));
-        if (dis < minDis) {
-            minDis = dis;
-            smin = s;
-            nel = elem1;
-        }
+    const int bj = (max(jm - 2, 1) - 1) / 4 + o % 3, bk = (max(km - 2, 1) - 1) / 4 + o / 3;
+    if (o >= 9 || bj > (min(jm + 3, ny + 2) - 1) / 4 || bk > (min(km + 3, nz + 2) - 1) / 4) return;
+    for (int bi = (i0 - 1) / 4; bi <= (i1 - 1) / 4; bi++) {
+        const int b = bi + (nx + 5) / 4 * (bj + (ny + 5) / 4 * bk);
+        // a relaxed load that already sees the flag skips the atomic (only the
+        // atomic that sets the flag queues the brick)
+        if (!__hip_atomic_load(bflag + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) && !atomicOr(bflag + b, 1u))
+            list[atomicAdd(count, 1)] = b;
     }
 }
 
@@ -263,72 +403,37 @@ __device__ __forceinline__ void retag_cell(int64_t c, int i, int j, int k, int n
 // 8-corner test, the same arithmetic as k_tagging.  A cell that was solid
 // and is no longer takes the wall velocity (the reference's body never
 // moves, so it has no rule for such cells).  Clears its queue flag.
-// A block takes 64 queued cells at a time; its 16 waves each scan one
-// contiguous slice of the elements (uniform loads), and wave 0 merges the
-// slices in element order with a strict '<', which gives the same first
-// nearest element as one pass over all of them.
-static constexpr int kRtSlices = 16;
-__global__ void __launch_bounds__(64 * kRtSlices)
-k_retag_list(const int *list, const int *count, int sx, int sy, const double *__restrict__ xp,
+// A workgroup takes a queued brick at a time, its four waves sharing the
+// clusters.
+__global__ void __launch_bounds__(256)
+k_retag_list(const int *list, const int *count, int sx, int sy, int sz, const double *__restrict__ xp,
              const double *__restrict__ yp, const double *__restrict__ zp, const double *__restrict__ x1,
              const double *__restrict__ y1, const double *__restrict__ z1, const double *__restrict__ xc,
              const double *__restrict__ yc, const double *__restrict__ zc, const double *__restrict__ ca,
-             const double *__restrict__ cb, const double *__restrict__ cg, int ne, int8_t *tag, int *minElem,
-             uint8_t *flag, double *u, double *v, double *w, double wu, double wv, double ww, int *err) {
-    __shared__ double s_dis[kRtSlices][64];
-    __shared__ int s_nel[kRtSlices][64];
+             const double *__restrict__ cb, const double *__restrict__ cg, ClusterView E, int8_t *tag, int *minElem,
+             uint8_t *flag, unsigned int *bflag, double *u, double *v, double *w, double wu, double wv, double ww,
+             int *err) {
     const int nq = *count;
-    const int lane = threadIdx.x & 63;
-    const int sl = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int chunk = (ne + kRtSlices - 1) / kRtSlices;
-    const int m0 = min(ne, sl * chunk), m1 = min(ne, m0 + chunk);
-    for (int q0 = blockIdx.x * 64; q0 < nq; q0 += gridDim.x * 64) {
-        const int q = q0 + lane;
-        const bool active = q < nq;
-        int i = 0, j = 0, k = 0;
-        int64_t c = 0;
-        if (active) {
-            c = list[q];
-            i = (int)(c % sx) + 1;
-            const int64_t r = c / sx;
-            j = (int)(r % sy) + 1;
-            k = (int)(r / sy) + 1;
-        }
-        const double n1x = active ? xp[i] : 0.0, n1y = active ? yp[j] : 0.0, n1z = active ? zp[k] : 0.0;
-        double minDis = 1e14, smin = __builtin_huge_val();
-        int nel = 0;
-        // four squared distances per step (their loads batch), then the
-        // updates in element order
-        int m = m0;
-        for (; m + 4 <= m1; m += 4) {
-            double s4[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const double dy = n1y - yc[m + t], dx = n1x - xc[m + t], dz = n1z - zc[m + t];
-                s4[t] = ((dy * dy) + (dx * dx)) + (dz * dz);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++) nearest_update(s4[t], m + t + 1, smin, minDis, nel);
-        }
-        for (; m < m1; m++) {
-            const double dy = n1y - yc[m], dx = n1x - xc[m], dz = n1z - zc[m];
-            nearest_update(((dy * dy) + (dx * dx)) + (dz * dz), m + 1, smin, minDis, nel);
-        }
-        s_dis[sl][lane] = minDis;
-        s_nel[sl][lane] = nel;
-        __syncthreads();
-        if (sl == 0 && active) {
-            for (int t = 1; t < kRtSlices; t++) {
-                const double d = s_dis[t][lane];
-                if (d < minDis) {
-                    minDis = d;
-                    nel = s_nel[t][lane];
-                }
-            }
-            retag_cell(c, i, j, k, nel, x1, y1, z1, xc, yc, zc, ca, cb, cg, tag, minElem, flag, u, v, w, wu, wv,
-                       ww, err);
-        }
-        __syncthreads();  // s_dis and s_nel are rewritten by the next group
+    const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int bx = (sx + 3) / 4, by = (sy + 3) / 4;
+    for (int q = blockIdx.x; q < nq; q += gridDim.x) {
+        const int b = list[q];
+        const int ib = 1 + 4 * (b % bx), jb = 1 + 4 * (b / bx % by), kb = 1 + 4 * (b / bx / by);
+        const int i = ib + (lane & 3), j = jb + ((lane >> 2) & 3), k = kb + (lane >> 4);
+        bool active = i <= sx && j <= sy && k <= sz;
+        const int64_t c = active ? lin(i, j, k, sx, sy) : 0;
+        active = active && flag[c];
+        double lo[3], hi[3];
+        axis_bounds(xp, ib, min(ib + 3, sx), lo[0], hi[0]);
+        axis_bounds(yp, jb, min(jb + 3, sy), lo[1], hi[1]);
+        axis_bounds(zp, kb, min(kb + 3, sz), lo[2], hi[2]);
+        const int nel = nearest_element<4>(E, active, active ? xp[i] : 0.0, active ? yp[j] : 0.0,
+                                           active ? zp[k] : 0.0, lo, hi, part);
+        // (nearest_element ends in a barrier: every wave has read the flags)
+        if (part == 0 && active)
+            retag_cell(c, i, j, k, nel, x1, y1, z1, xc, yc, zc, ca, cb, cg, tag, minElem, flag, u, v, w, wu, wv, ww,
+                       err);
+        if (threadIdx.x == 0) bflag[b] = 0;
     }
 }
 
@@ -871,33 +976,91 @@ void ib_release() {
 
 int count_tags(Ctx &c, int32_t out[4], bool scatter);
 
+// The cluster order of a mesh: elements along a Morton curve through the
+// bounding box of their centroids (any order gives the same tags; a compact
+// one lets more clusters be skipped), the last cluster padded with -1.
+int set_clusters(Ctx &c, const double *xn, const double *yn, const double *zn, const int *elp, int64_t ne) {
+    const double *node[3] = {xn, yn, zn};
+    std::vector<float> pos(3 * ne);
+    float lo[3], inv[3];
+    for (int a = 0; a < 3; a++) {
+        float mn = HUGE_VALF, mx = -HUGE_VALF;
+        for (int64_t e = 0; e < ne; e++) {
+            const float v = (float)((node[a][elp[e] - 1] + node[a][elp[ne + e] - 1] + node[a][elp[2 * ne + e] - 1]) / 3.0);
+            pos[a * ne + e] = v;
+            mn = std::min(mn, v);   // (a NaN is ignored)
+            mx = std::max(mx, v);
+        }
+        lo[a] = mn;
+        inv[a] = mx > mn && std::isfinite(mx - mn) ? 1023.0f / (mx - mn) : 0.0f;
+    }
+    std::vector<uint64_t> key(ne);   // Morton code above the element
+    for (int64_t e = 0; e < ne; e++) {
+        uint64_t code = 0;
+        for (int a = 0; a < 3; a++) {
+            const float f = (pos[a * ne + e] - lo[a]) * inv[a];
+            uint64_t v = f >= 0.0f ? (uint64_t)std::min(f, 1023.0f) : 0;
+            for (int bit = 0; bit < 10; bit++) code |= ((v >> bit) & 1) << (3 * bit + a);
+        }
+        key[e] = code << 32 | (uint64_t)e;
+    }
+    std::sort(key.begin(), key.end());
+    const int64_t nc = (ne + kCluster - 1) / kCluster;
+    std::vector<int> perm(nc * kCluster, -1);
+    for (int64_t e = 0; e < ne; e++) perm[e] = (int)(key[e] & 0xffffffffu);
+    release_clusters(c);
+    IB3D_CHECK(hipMalloc(&c.cl_perm, perm.size() * sizeof(int)));
+    IB3D_CHECK(hipMalloc(&c.cl_id, perm.size() * sizeof(int)));
+    IB3D_CHECK(hipMalloc(&c.cl_pos, 3 * perm.size() * sizeof(double)));
+    IB3D_CHECK(hipMalloc(&c.cl_box, 6 * nc * sizeof(double)));
+    IB3D_CHECK(h2d(c.cl_perm, perm.data(), perm.size() * sizeof(int)));
+    c.n_clusters = nc;
+    return 0;
+}
+
+void release_clusters(Ctx &c) {
+    if (c.cl_perm) (void)hipFree(c.cl_perm);
+    if (c.cl_id) (void)hipFree(c.cl_id);
+    if (c.cl_pos) (void)hipFree(c.cl_pos);
+    if (c.cl_box) (void)hipFree(c.cl_box);
+    c.cl_perm = c.cl_id = nullptr;
+    c.cl_pos = c.cl_box = nullptr;
+    c.n_clusters = 0;
+}
+
+// the clusters of the current centroids
+static ClusterView clusters(Ctx &c) {
+    const int nc = (int)c.n_clusters;
+    hipLaunchKernelGGL(k_clusters, dim3(nblocks(nc, 4)), dim3(256), 0, c.stream, c.cl_perm, c.xcent, c.ycent,
+                       c.zcent, nc, c.cl_pos, c.cl_id, c.cl_box);
+    return ClusterView{c.cl_pos, c.cl_box, c.cl_id, nc};
+}
+
 // subSearch.f90:327-463 selectiveRetagging
 int selective_retagging(Ctx &c, int32_t counts[3]) {
     IB3D_REQUIRE(c.norms_ready, "selectiveRetagging: computeSurfaceNorm has not run");
     IB3D_REQUIRE(c.lists_ready, "selectiveRetagging: cellCount has not run");
     const int64_t nb = c.ibCount;
+    const int64_t cap = ((c.sx + 3) / 4) * ((c.sy + 3) / 4) * ((c.sz + 3) / 4);   // bricks of the grid
     if (!c.rt_flag) {
-        IB3D_CHECK(hipMalloc(&c.rt_flag, (c.P + 4) * sizeof(uint8_t)));
-        IB3D_CHECK(hipMemsetAsync(c.rt_flag, 0, (c.P + 4) * sizeof(uint8_t), c.stream));
-        IB3D_CHECK(hipMalloc(&c.rt_count, sizeof(int)));
-    }
-    const int64_t cap = std::min<int64_t>(c.P, std::max<int64_t>(1, 216 * nb));
-    if (cap > c.rt_cap) {
-        IB3D_CHECK(hipStreamSynchronize(c.stream));
-        if (c.rt_list) IB3D_CHECK(hipFree(c.rt_list));
+        IB3D_CHECK(hipMalloc(&c.rt_bflag, cap * sizeof(unsigned int)));
+        IB3D_CHECK(hipMemsetAsync(c.rt_bflag, 0, cap * sizeof(unsigned int), c.stream));
         IB3D_CHECK(hipMalloc(&c.rt_list, cap * sizeof(int)));
-        c.rt_cap = cap;
+        IB3D_CHECK(hipMalloc(&c.rt_count, sizeof(int)));
+        IB3D_CHECK(hipMalloc(&c.rt_flag, c.P * sizeof(uint8_t)));
+        IB3D_CHECK(hipMemsetAsync(c.rt_flag, 0, c.P * sizeof(uint8_t), c.stream));
     }
     IB3D_CHECK(hipMemsetAsync(c.minElem, 0, c.P * sizeof(int), c.stream));
     IB3D_CHECK(hipMemsetAsync(c.rt_count, 0, sizeof(int), c.stream));
     if (dev_err(c)) return -1;
     if (nb > 0) {
-        hipLaunchKernelGGL(k_retag_mark, dim3(nblocks(216 * nb, 1024)), dim3(1024), 0, c.stream, c.ibList, (int)nb,
-                           (int)c.nx, (int)c.ny, (int)c.nz, c.rt_flag, c.rt_list, c.rt_count);
-        const unsigned grid = (unsigned)std::min<int64_t>(nblocks(cap, 64), 1024);
-        hipLaunchKernelGGL(k_retag_list, dim3(grid), dim3(64 * kRtSlices), 0, c.stream, c.rt_list,
-                           c.rt_count, (int)c.sx, (int)c.sy, c.xp, c.yp, c.zp, c.x1, c.y1, c.z1, c.xcent, c.ycent,
-                           c.zcent, c.cosA, c.cosB, c.cosG, (int)c.ibElems, c.tag, c.minElem, c.rt_flag, c.u, c.v,
+        hipLaunchKernelGGL(k_retag_mark, dim3(nblocks(36 * nb, 256)), dim3(256), 0, c.stream, c.ibList, (int)nb,
+                           (int)c.nx, (int)c.ny, (int)c.nz, c.rt_flag, c.rt_bflag, c.rt_list, c.rt_count);
+        const ClusterView cl = clusters(c);
+        const unsigned grid = (unsigned)std::min<int64_t>(cap, 4096);
+        hipLaunchKernelGGL(k_retag_list, dim3(grid), dim3(256), 0, c.stream, c.rt_list,
+                           c.rt_count, (int)c.sx, (int)c.sy, (int)c.sz, c.xp, c.yp, c.zp, c.x1, c.y1, c.z1, c.xcent, c.ycent,
+                           c.zcent, c.cosA, c.cosB, c.cosG, cl, c.tag, c.minElem, c.rt_flag, c.rt_bflag, c.u, c.v,
                            c.w, c.wall_vel[0], c.wall_vel[1], c.wall_vel[2], g_err);
     }
     IB3D_CHECK(hipGetLastError());
@@ -921,11 +1084,13 @@ int tagging(Ctx &c, const int64_t w[6], int32_t counts[3]) {
     IB3D_CHECK(hipMemsetAsync(c.tag, 0, c.P, c.stream));
     IB3D_CHECK(hipMemsetAsync(c.minElem, 0, c.P * sizeof(int), c.stream));
     if (dev_err(c)) return -1;
-    const int64_t nw = (w[1] - w[0] + 1) * (w[3] - w[2] + 1) * (w[5] - w[4] + 1);
-    hipLaunchKernelGGL(k_tagging, dim3(nblocks(nw, kTagTile)), dim3(kTagTile), 0, c.stream, (int)w[0], (int)w[1],
-                       (int)w[2], (int)w[3], (int)w[4], (int)w[5], (int)c.sx, (int)c.sy, c.xp, c.yp, c.zp, c.x1,
-                       c.y1, c.z1, c.xcent, c.ycent, c.zcent, c.cosA, c.cosB, c.cosG, (int)c.ibElems, c.tag,
-                       c.minElem, g_err);
+    const int64_t nb = ((w[1] - w[0] + 4) / 4) * ((w[3] - w[2] + 4) / 4) * ((w[5] - w[4] + 4) / 4);
+    const ClusterView cl = clusters(c);
+    const bool few = nb < 8192;
+    hipLaunchKernelGGL(few ? k_tagging<4> : k_tagging<1>, dim3(nblocks(few ? 4 * nb : nb, kTagTile / 64)),
+                       dim3(kTagTile), 0, c.stream, (int)w[0], (int)w[1], (int)w[2], (int)w[3], (int)w[4],
+                       (int)w[5], (int)c.sx, (int)c.sy, c.xp, c.yp, c.zp, c.x1, c.y1, c.z1, c.xcent, c.ycent,
+                       c.zcent, c.cosA, c.cosB, c.cosG, cl, c.tag, c.minElem, g_err);
     IB3D_CHECK(hipGetLastError());
     IB3D_REQUIRE(read_err(c, g_err) == 0, "tagging: a window cell found no element closer than 1e14");
     int32_t t4[4];

@@ -126,6 +126,11 @@ struct Ctx {
     double *cosA = nullptr, *cosB = nullptr, *cosG = nullptr;
     double *alpha3 = nullptr, *beta3 = nullptr, *gamma3 = nullptr;
     bool norms_ready = false;
+    // clusters of 64 neighbouring elements: their order (once per mesh), and
+    // the centroids in that order with each cluster's box (per search)
+    int *cl_perm = nullptr, *cl_id = nullptr;
+    double *cl_pos = nullptr, *cl_box = nullptr;
+    int64_t n_clusters = 0;
 
     // lists: int32 SoA [3][count], (k,j,i) order like the reference
     int64_t ibCount = 0, fluidCount = 0, solidCount = 0, redCount = 0, blackCount = 0;
@@ -151,10 +156,10 @@ struct Ctx {
     // forcing, the solid cells and the surface forces; body acceleration
     // for dp/dn at the wall; retagging scratch
     double wall_vel[3] = {0.0, 0.0, 0.0}, wall_acc[3] = {0.0, 0.0, 0.0};
-    uint8_t *rt_flag = nullptr;    // P flags: cell queued for retagging
-    int *rt_list = nullptr;        // unique queued cells (linear index)
+    uint8_t *rt_flag = nullptr;        // P flags: cell to be retagged
+    unsigned int *rt_bflag = nullptr;  // per 4x4x4 brick: queued
+    int *rt_list = nullptr;            // queued bricks
     int *rt_count = nullptr;
-    int64_t rt_cap = 0;
 
     // Poisson configuration
     int mode = 0;                  // 0 reference rule, 1 FP64 L2, 2 mixed FP32/FP64, 3 FP32 GMRES in FP64 refinement, 4 the same with a multigrid preconditioner
@@ -295,6 +300,8 @@ int64_t resid_guard_selfcheck(int64_t nx, int64_t ny, int64_t nz, bool drop_inte
 int set_momentum_tiles(int on);
 int redblack_sor_reference(Ctx &c, double epsi, int64_t *isum, double *derr2);
 int plans_launch(Ctx &c);
+int set_clusters(Ctx &c, const double *xn, const double *yn, const double *zn, const int *elp, int64_t ne);
+void release_clusters(Ctx &c);
 int shift_nodes_moving(Ctx &c, const double base[3], const double disp[3]);
 int selective_retagging(Ctx &c, int32_t counts[3]);
 int stress_bodies(Ctx &c, double *coef);
