@@ -20,9 +20,9 @@
 //             pair also supplies the x neighbours); colour rows have even
 //             length so every pair is an aligned vector access, and the
 //             coefficients are hoisted out of the z loop.
-//   k_sor_block  (ib3d_sor_block.h) two whole sweeps of a block of cells in one
-//             launch, out of registers and LDS: grids up to 1.5 M cells (FP64)
-//             and 2 M (FP32) in modes 0 to 3.
+//   k_sor_block, k_sor_march  (ib3d_sor_block.h, ib3d_sor_march.h) two whole
+//             sweeps in one launch, out of registers and LDS: the sweeps of all
+//             modes, on small and on large grids (sweep_plan).
 //   k_sor     one cell per thread: the smoother on the coarse multigrid
 //             levels, where a z-marching thread would have too few peers.
 //   k_resid_pz  FP64 residual b/dt - A p over both colours (optionally of
@@ -219,6 +219,7 @@ __device__ __forceinline__ double sor_div(double a, double b) { return a / b; }
 __device__ __forceinline__ float sor_div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 
 #include "ib3d_sor_block.h"
+#include "ib3d_sor_march.h"
 
 // One colour half-sweep, one cell per thread.
 // FIRST: the unknown starts from zero (own old value and, for the red
@@ -352,7 +353,8 @@ k_sor_pz(T *__restrict__ mine, const T *__restrict__ other, const T *__restrict_
     if (TRACK) block_max_to(d, slot);
 }
 
-// One whole FP32 red-black sweep in one launch (the finest multigrid level).
+// One whole FP32 red-black sweep in one launch (multigrid levels with a launch
+// shape of the caller's, and sweeps that pairs leave over).
 // Red is updated from the old black values, black from the new red values,
 // exactly as two half-sweeps in place, but the result goes to a second
 // buffer: red_new/black_new are written to dst while src keeps the old values,
@@ -565,125 +567,6 @@ k_sweep2_pz(const float *__restrict__ src0, const float *__restrict__ src1, floa
         march(std::true_type{});
     else
         march(std::false_type{});
-}
-
-// Several red-black sweeps of a coarse multigrid level in one launch
-// (temporal blocking).  A workgroup owns a CX x CY x CZ block of cells (8 x 8
-// x 8 as launched) and loads it into LDS with a halo of 2M cells on every
-// side (M sweeps: each half-sweep moves the dependency one cell), in natural
-// (i, j, k) order, both colours interleaved.  Half-sweep m (1..2M) updates
-// the cells of its colour that lie at most 2M-m cells outside the block, so
-// the values it reads were exact after half-sweep m-1 and the block is exact
-// after the last one.  The block's
-// interior cells (both colours: updated cells and, copied through, the cells
-// outside the solve) go to dst, never to src, which the neighbouring
-// workgroups are still reading; walls are never written (they stay as in
-// src).  Positions outside the arrays hold 0 and a NaN right-hand side, so
-// they are never updated and only wall cells read them.  FIRST: the first
-// red half-sweep takes every neighbour and the old value as 0, and the first
-// black half-sweep the old value, as k_sor does from zero.  Every update is
-// k_sor's, operand for operand: the result is bit for bit that of 2M
-// half-sweep launches.
-static constexpr int kTileCube = 8;       // the cube of levels 2 and below
-static constexpr int kTileMaxSweeps = 2;
-static constexpr int kTileThreads = 1024;
-template <bool FIRST, int M, int CX, int CY, int CZ>
-__global__ void __launch_bounds__(kTileThreads)
-k_smooth_tile(const float *__restrict__ src, float *__restrict__ dst, const float *__restrict__ b,
-              const float *__restrict__ axc, const float *__restrict__ ayc, const float *__restrict__ azc, SorGeom g,
-              float omega, float omm, const double *gate, double thr) {
-    static_assert(M >= 1 && M <= kTileMaxSweeps, "sweeps per launch");
-    constexpr int R = 2 * M, EX = CX + 2 * R, EY = CY + 2 * R, EZ = CZ + 2 * R;
-    constexpr int E2 = EX * EY, E3 = E2 * EZ;
-    __shared__ float xs[E3];
-    __shared__ float bs[E3];
-    __shared__ float cx[3][EX], cy[3][EY], cz[3][EZ];
-    if (gated(gate, thr)) return;
-    // cuboid origin (first interior cell) minus the halo: tile position 0
-    const int i0 = 1 + CX * (int)blockIdx.x - R;
-    const int j0 = 1 + CY * (int)blockIdx.y - R;
-    const int k0 = 1 + CZ * (int)blockIdx.z - R;
-    const int tid = (int)threadIdx.x;
-    const float nan = __builtin_nanf("");
-    // coefficient rows of the tile's columns (clamped: positions outside
-    // the arrays are never updated, so their rows are never used)
-    const int ax_ = min(tid / EX, 2), tx_ = tid - ax_ * EX;
-    const int ay_ = min(tid / EY, 2), ty_ = tid - ay_ * EY;
-    const int az_ = min(tid / EZ, 2), tz_ = tid - az_ * EZ;
-    float cxv = 0.0f, cyv = 0.0f, czv = 0.0f;
-    if (tid < 3 * EX) cxv = axc[ax_ * g.sxp + min(max(i0 + tx_, 0), g.sx - 1)];
-    if (tid < 3 * EY) cyv = ayc[ay_ * g.sy + min(max(j0 + ty_, 0), g.sy - 1)];
-    if (tid < 3 * EZ) czv = azc[az_ * g.sz + min(max(k0 + tz_, 0), g.sz - 1)];
-    // every thread issues all of its loads (at most kTileLoads cells each)
-    // before it stores any, so their latencies overlap; positions outside the
-    // arrays load a clamped (valid) cell and store 0 and NaN instead
-    constexpr int kTileLoads = (E3 + kTileThreads - 1) / kTileThreads;
-    float xv[kTileLoads], bv[kTileLoads];
-    bool in[kTileLoads];
-#pragma unroll
-    for (int q = 0; q < kTileLoads; q++) {
-        const int n = min(tid + q * kTileThreads, E3 - 1);
-        const int lk = n / E2, r = n - lk * E2, lj = r / EX, li = r - lj * EX;
-        const int ii = i0 + li, jj = j0 + lj, kk = k0 + lk;
-        in[q] = ii >= 0 && ii < g.sx && jj >= 0 && jj < g.sy && kk >= 0 && kk < g.sz;
-        const int ic = min(max(ii, 0), g.sx - 1), jc = min(max(jj, 0), g.sy - 1), kc = min(max(kk, 0), g.sz - 1);
-        const uint32_t f = (uint32_t)((kc * g.sy + jc) * g.H + (ic >> 1) + ((ic + jc + kc) & 1) * g.NC);
-        bv[q] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + f * 4u);
-        xv[q] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(src) + f * 4u);
-    }
-#pragma unroll
-    for (int q = 0; q < kTileLoads; q++) {
-        const int n = tid + q * kTileThreads;
-        if (n < E3) {
-            const float bq = in[q] ? bv[q] : nan;
-            xs[n] = in[q] ? ((FIRST && bq == bq) ? 0.0f : xv[q]) : 0.0f;
-            bs[n] = bq;
-        }
-    }
-    if (tid < 3 * EX) cx[ax_][tx_] = cxv;
-    if (tid < 3 * EY) cy[ay_][ty_] = cyv;
-    if (tid < 3 * EZ) cz[az_][tz_] = czv;
-    __syncthreads();
-#pragma unroll
-    for (int m = 1; m <= 2 * M; m++) {
-        const int col = (m - 1) & 1;
-        // region [m, E-m) per axis; cells of one colour per row <= HW
-        const int WX = EX - 2 * m, WY = EY - 2 * m, WZ = EZ - 2 * m, HW = (WX + 1) >> 1;
-#pragma unroll
-        for (int idx = tid; idx < HW * WY * WZ; idx += kTileThreads) {
-            const int row = idx / HW, p = idx - row * HW;
-            const int lk = m + row / WY, lj = m + (row - (row / WY) * WY);
-            const int li = m + (((col - (i0 + m + j0 + lj + k0 + lk)) & 1)) + 2 * p;
-            if (li >= EX - m) continue;
-            const int n = li + EX * (lj + EY * lk);
-            const float r = bs[n];
-            if (!(r == r)) continue;
-            float pw, pe, ps, pn, pb, pt;
-            if (FIRST && m == 1) {
-                pw = pe = ps = pn = pb = pt = 0.0f;
-            } else {
-                pw = xs[n - 1]; pe = xs[n + 1];
-                ps = xs[n - EX]; pn = xs[n + EX];
-                pb = xs[n - E2]; pt = xs[n + E2];
-            }
-            const float pold = xs[n];
-            const float a1x = cx[0][li], a2x = cx[1][li], a3x = cx[2][li];
-            const float a1y = cy[0][lj], a2y = cy[1][lj], a3y = cy[2][lj];
-            const float a1z = cz[0][lk], a2z = cz[1][lk], a3z = cz[2][lk];
-            const float gs = sor_div(((((((r - a1x * pw) - a3x * pe) - a1y * ps) - a3y * pn) - a1z * pb) - a3z * pt),
-                                     ((a2x + a2y) + a2z));
-            xs[n] = omm * pold + omega * gs;
-        }
-        __syncthreads();
-    }
-    for (int n = tid; n < CX * CY * CZ; n += kTileThreads) {
-        const int ck = n / (CX * CY), r = n - ck * CX * CY, cj = r / CX, ci = r - cj * CX;
-        const int li = R + ci, lj = R + cj, lk = R + ck;
-        const int ii = i0 + li, jj = j0 + lj, kk = k0 + lk;
-        if (ii > g.sx - 2 || jj > g.sy - 2 || kk > g.sz - 2) continue;
-        const int f = (kk * g.sy + jj) * g.H + (ii >> 1) + ((ii + jj + kk) & 1) * g.NC;
-        dst[f] = xs[li + EX * (lj + EY * lk)];
-    }
 }
 
 // FP64 residual r = b/dt - A p over both colours.  ADD: of p + e (e is the
@@ -1526,19 +1409,23 @@ static dim3 pz_grid(const Ctx &c) {
     return dim3(nblocks((c.H * c.sy) / 2, kSorBlock), (unsigned)((c.sz - 2 + kZch - 1) / kZch));
 }
 
-// FP64 sweep (both colours) gated on *gate < thr
-static void sweep64(Ctx &c, double omega, bool track, double *slot, const double *gate, double thr) {
+// FP64 sweep (both colours) of p in place, gated on *gate < thr
+static void sweep64_on(Ctx &c, double *const p[2], double omega, bool track, double *slot, const double *gate,
+                       double thr) {
     const SorGeom g = geom(c);
     for (int col = 0; col < 2; col++) {
         if (track)
             hipLaunchKernelGGL((k_sor_pz<double, true, false, false>), pz_grid(c), dim3(kSorBlock), 0, c.stream,
-                               c.pc[col], c.pc[1 - col], c.bdt[col], c.ax, c.ay, c.az, g, col, omega, 1.0 - omega,
+                               p[col], p[1 - col], c.bdt[col], c.ax, c.ay, c.az, g, col, omega, 1.0 - omega,
                                slot, gate, thr, nullptr);
         else
             hipLaunchKernelGGL((k_sor_pz<double, false, false, false>), pz_grid(c), dim3(kSorBlock), 0, c.stream,
-                               c.pc[col], c.pc[1 - col], c.bdt[col], c.ax, c.ay, c.az, g, col, omega, 1.0 - omega,
+                               p[col], p[1 - col], c.bdt[col], c.ax, c.ay, c.az, g, col, omega, 1.0 - omega,
                                slot, gate, thr, nullptr);
     }
+}
+static void sweep64(Ctx &c, double omega, bool track, double *slot, const double *gate, double thr) {
+    sweep64_on(c, c.pc, omega, track, slot, gate, thr);
 }
 
 // FP32 sweep (both colours) on the increment e; first: start from zero,
@@ -1627,21 +1514,110 @@ static int second_e(Ctx &c) {
     return 0;
 }
 
-// Block shapes by grid size.  A CU works on one block of 24 x 16 x 8 (98 KB of
-// LDS in FP64) or a few small ones, so a small grid wants blocks small enough
-// to reach every CU, and a large one blocks with little halo.  us per FP64
-// sweep (TRACK) on 8x8x4 | 8x8x8 | 24x16x8 blocks and with half-sweep launches:
-// 18k cells 3.5 | 4.3 | 6.5 | 14.9, 49k 4.1 | 4.4 | 6.5 | 17.6, 147k
-// 6.3 | 6.0 | 6.9 | 17.8, 301k 10.0 | 7.7 | 7.5 | 18.7, 524k 14.9 | 11.2 | 8.2 |
-// 16.5, 1.47M - | 22.3 | 15.1 | 20.1, 1.70M - | 27.5 | 20.9 | 21.3.  FP32 on
-// 24x8x8: 3.0-3.3 up to 147k, 4.8 at 524k, 8.3 at 1.47M, 9.9 at 1.70M (half-
-// sweeps 11.6-15.5).
-enum { kBlockNone = 0, kBlock884, kBlock888, kBlock24168, kBlock2488 };
-static int block_shape(const Ctx &c, bool fp64) {
-    const int64_t cells = c.nx * c.ny * c.nz;
-    if (c.NC >= (int64_t)1 << 28) return kBlockNone;   // 32-bit byte offsets into a colour array
-    if (!fp64) return cells <= 2000000 ? kBlock2488 : kBlockNone;
-    if (cells > 1500000) return kBlockNone;
+// ---- which launches sweep a grid
+// A plan: one of k_sor_block's shapes or k_sor_march's tiles, by grid size.
+//
+// Blocks: a CU works on one block of 24 x 16 x 8 (98 KB of LDS in FP64) or a few
+// small ones, so a small grid wants blocks small enough to reach every CU, and a
+// larger one blocks with little halo; the march, whose tiles read 1.6 times
+// their cells instead of a block's four times, wins where it has enough planes
+// per chunk.  us per FP64 sweep (TRACK), half-sweep launches | 8x8x4 | 8x8x8 |
+// 24x16x8 | march:
+//   18k cells  14.9 |  3.5 |  4.3 |  6.5 |           49k  17.6 |  4.1 |  4.4 |  6.5 |
+//   147k       17.8 |  6.3 |  6.0 |  6.9 |           301k 18.7 | 10.0 |  7.7 |  7.5 |
+//   524k       16.5 | 14.9 | 11.2 |  8.2 | 11.4      1.47M 20.1 |     | 22.3 | 15.1 | 16.8
+//   1.70M      21.3 |      | 27.5 | 20.9 | 17.9      9.4M  66.8 |     |      |      | 44.0
+//   25M       180.0 |      |      |      | 98.9
+// and per FP32 sweep, half-sweep launches | 8x8x4 | 24x8x8 | march:
+//   18k  11.7 | 2.6 |  3.1 |        66k  16.1 | 2.8 |  3.2 |  5.0     147k 14.9 | 3.6 | 3.4 | 5.1
+//   524k 12.7 | 6.8 |  4.8 |  6.0   819k 16.5 |     |  6.7 |  6.7     1.2M 16.5 |    | 8.1 | 7.2
+//   1.7M 15.4 |     |  9.9 |  7.8   3.1M 15.9 |     | 14.4 | 10.0     9.4M 29.0 |  | 38.4 | 18.6
+//   25M  63.7 |     |      | 46.8   52M  181  |     |      | 83.8
+enum SweepKind { kPlanNone = 0, kBlock884, kBlock888, kBlock24168, kBlock2488, kMarch3628, kMarch3232 };
+struct SweepPlan {
+    SweepKind kind = kPlanNone;
+    int64_t NC = 0;
+    SorGeom g{};
+    int n0 = 0, n1 = 0, tz = 0;   // blocks or tiles in x and y; planes per chunk of the march
+    unsigned wgs = 0;
+    bool march() const { return kind >= kMarch3628; }
+    // whether n sweeps hold an even number of launches (a -> b -> a ends where it
+    // began): blocks do two sweeps or one, the march always two
+    bool pays(int n) const { return kind && n >= (march() ? 4 : 2); }
+    // sweeps left to other launches (done first)
+    int alone(int n) const { return march() ? n % 4 : 0; }
+    // the launches of n sweeps (n - alone): f(sweeps, launch index)
+    template <typename F> void launches(int n, F f) const {
+        if (!kind || n <= 0) return;
+        int two = n / 2, one = n % 2;
+        if ((two + one) % 2) {
+            two--;
+            one += 2;
+        }
+        for (int q = 0; q < two + one; q++) f(q < two ? 2 : 1, q);
+    }
+};
+
+// k_sor_march's tiles along x (of `len` interior cells) and y; the end tiles need
+// no halo outside the grid
+static int march_tiles_x(int hx, int64_t nx) {
+    const int64_t ns = nx / 2 + 1;
+    return ns <= hx - 1 ? 1 : (int)std::max<int64_t>(2, 2 + (ns - (2 * hx - 5) + hx - 5) / (hx - 4));
+}
+static int march_tiles_y(int ey, int64_t ny) {
+    return ny + 2 <= ey ? 1 : (int)std::max<int64_t>(2, 2 + (ny - (2 * ey - 10) + ey - 9) / (ey - 8));
+}
+
+static SweepPlan sweep_plan(int64_t nx, int64_t ny, int64_t nz, int64_t NC, const SorGeom &g, bool fp64) {
+    SweepPlan P;
+    const int64_t cells = nx * ny * nz;
+    if (NC >= (int64_t)1 << 28) return P;   // 32-bit byte offsets into a colour array
+    P.NC = NC;
+    P.g = g;
+    if (cells > (fp64 ? 1500000 : 800000)) {
+        // one workgroup per CU: the chunk count with the fewest steps (a chunk of
+        // tz planes marches tz + 8), over both tile shapes
+        const int shape[2][2] = {{32, 32}, {36, 28}};
+        double best = HUGE_VAL;
+        for (int q = 0; q < 2; q++) {
+            const int tx = march_tiles_x(shape[q][0], nx), ty = march_tiles_y(shape[q][1], ny);
+            for (int64_t n = 1; n <= std::min<int64_t>(nz, 256); n++) {
+                const int64_t tz = (nz + n - 1) / n, wgs = (int64_t)tx * ty * ((nz + tz - 1) / tz);
+                const double cost = (double)((wgs + 255) / 256) * (double)(tz + 8);
+                if (cost < best) {
+                    best = cost;
+                    P.kind = q ? kMarch3628 : kMarch3232;
+                    P.n0 = tx;
+                    P.n1 = ty;
+                    P.tz = (int)tz;
+                    P.wgs = (unsigned)wgs;
+                }
+            }
+        }
+        return P;
+    }
+    int bx = 8, by = 8, bz = 8;
+    if (cells <= 65536) {
+        P.kind = kBlock884;
+        bz = 4;
+    } else if (!fp64) {
+        P.kind = kBlock2488;
+        bx = 24;
+    } else if (cells <= 262144) {
+        P.kind = kBlock888;
+    } else {
+        P.kind = kBlock24168;
+        bx = 24;
+        by = 16;
+    }
+    P.n0 = (int)((nx + bx - 1) / bx);
+    P.n1 = (int)((ny + by - 1) / by);
+    P.wgs = (unsigned)(P.n0 * P.n1 * ((nz + bz - 1) / bz));
+    return P;
+}
+
+static SweepPlan plan32(const Ctx &c) { return sweep_plan(c.nx, c.ny, c.nz, c.NC, geom(c), false); }
+static SweepPlan plan64(const Ctx &c) {
     // block_div's denominators: every diagonal in [-2^64, -2^-64], as any grid
     // of non-extreme spacings gives (the sums of the axes' extremes bound them)
     double lo = 0.0, hi = 0.0;
@@ -1651,89 +1627,91 @@ static int block_shape(const Ctx &c, bool fp64) {
         double mn = HUGE_VAL, mx = -HUGE_VAL;
         for (int64_t i = 0; i < n[a]; i++) {
             const double v = (*A[a])[i + n[a]];
-            if (!std::isfinite(v)) return kBlockNone;
+            if (!std::isfinite(v)) return SweepPlan{};
             mn = std::min(mn, v);
             mx = std::max(mx, v);
         }
         lo += mn;
         hi += mx;
     }
-    if (!(hi <= -0x1p-64 && lo >= -0x1p64)) return kBlockNone;
-    return cells <= 65536 ? kBlock884 : cells <= 262144 ? kBlock888 : kBlock24168;
+    if (!(hi <= -0x1p-64 && lo >= -0x1p64)) return SweepPlan{};
+    return sweep_plan(c.nx, c.ny, c.nz, c.NC, geom(c), true);
 }
 
-template <typename T, int M, int OX, int OY, int OZ, bool FIRST, bool TRACK, bool APPLY>
-static void launch_block(Ctx &c, const T *s0, const T *s1, T *d0, T *d1, const T *r0, const T *r1, const T *ax,
-                         const T *ay, const T *az, T omega, T omm, const double *gate, double thr,
-                         const double *prev, double *slot, double *acc0, double *acc1) {
-    const int nbx = (int)((c.nx + OX - 1) / OX), nby = (int)((c.ny + OY - 1) / OY), nbz = (int)((c.nz + OZ - 1) / OZ);
-    hipLaunchKernelGGL((k_sor_block<T, M, OX, OY, OZ, FIRST, TRACK, APPLY>), dim3((unsigned)(nbx * nby * nbz)),
-                       dim3((BlockShape<M, OX, OY, OZ>::NT)), 0, c.stream, s0, s1, d0, d1, r0, r1, ax, ay, az,
-                       geom(c), nbx, nby, omega, omm, gate, thr, prev, slot, acc0, acc1);
+// M sweeps, (s0, s1) -> (d0, d1)
+template <typename T, int M, bool FIRST, bool TRACK, bool APPLY>
+static void launch_sweeps(Ctx &c, const SweepPlan &P, const T *s0, const T *s1, T *d0, T *d1, const T *r0,
+                          const T *r1, const T *ax, const T *ay, const T *az, T omega, T omm, const double *gate,
+                          double thr, const double *prev, double *slot, double *acc0, double *acc1) {
+#define IB3D_BLOCK(X, Y, Z)                                                                                         \
+    hipLaunchKernelGGL((k_sor_block<T, M, X, Y, Z, FIRST, TRACK, APPLY>), dim3(P.wgs),                               \
+                       dim3((BlockShape<M, X, Y, Z>::NT)), 0, c.stream, s0, s1, d0, d1, r0, r1, ax, ay, az, P.g,     \
+                       P.n0, P.n1, omega, omm, gate, thr, prev, slot, acc0, acc1)
+#define IB3D_MARCH(HX, EY)                                                                                          \
+    hipLaunchKernelGGL((k_sor_march<T, HX, EY, FIRST, TRACK, APPLY>), dim3(P.wgs), dim3((MarchShape<HX, EY>::NT)),   \
+                       0, c.stream, s0, s1, d0, d1, r0, r1, ax, ay, az, P.g, P.n0, P.n1, P.tz, omega, omm, gate,     \
+                       thr, prev, slot, acc0, acc1)
+    if (P.kind == kBlock884) IB3D_BLOCK(8, 8, 4);
+    else if constexpr (sizeof(T) == 8) {
+        if (P.kind == kBlock888) IB3D_BLOCK(8, 8, 8);
+        else if (P.kind == kBlock24168) IB3D_BLOCK(24, 16, 8);
+    } else if (P.kind == kBlock2488) IB3D_BLOCK(24, 8, 8);
+    if constexpr (M == 2) {
+        if (P.kind == kMarch3628) IB3D_MARCH(36, 28);
+        else if (P.kind == kMarch3232) IB3D_MARCH(32, 32);
+    }
+#undef IB3D_MARCH
+#undef IB3D_BLOCK
 }
 
 // M (1 or 2) FP64 sweeps between pc (buffer 0) and g_pc2 (buffer 1), from
 // buffer `from`; TRACK (M = 2) when slot is given
-static void block64(Ctx &c, int shape, int M, int from, double omega, const double *gate, double thr,
-                    const double *prev = nullptr, double *slot = nullptr) {
+static void launch64(Ctx &c, const SweepPlan &P, int M, int from, double omega, const double *gate, double thr,
+                     const double *prev = nullptr, double *slot = nullptr) {
     double *b[2][2] = {{c.pc[0], c.pc[1]}, {g_pc2, g_pc2 + c.NC}};
     double **s = b[from], **d = b[1 - from];
-    const double omm = 1.0 - omega;
-#define IB3D_BLOCK(MM, TR, X, Y, Z)                                                                                 \
-    launch_block<double, MM, X, Y, Z, false, TR, false>(c, s[0], s[1], d[0], d[1], c.bdt[0], c.bdt[1], c.ax, c.ay,   \
-                                                        c.az, omega, omm, gate, thr, prev, slot, nullptr, nullptr)
-#define IB3D_SHAPES(MM, TR)                                                                                         \
-    do {                                                                                                            \
-        if (shape == kBlock884) IB3D_BLOCK(MM, TR, 8, 8, 4);                                                        \
-        else if (shape == kBlock888) IB3D_BLOCK(MM, TR, 8, 8, 8);                                                   \
-        else IB3D_BLOCK(MM, TR, 24, 16, 8);                                                                         \
-    } while (0)
-    if (slot) IB3D_SHAPES(2, true);
-    else if (M == 2) IB3D_SHAPES(2, false);
-    else IB3D_SHAPES(1, false);
-#undef IB3D_SHAPES
-#undef IB3D_BLOCK
+#define IB3D_SWEEPS(MM, TR)                                                                                         \
+    launch_sweeps<double, MM, false, TR, false>(c, P, s[0], s[1], d[0], d[1], c.bdt[0], c.bdt[1], c.ax, c.ay, c.az,  \
+                                                omega, 1.0 - omega, gate, thr, prev, slot, nullptr, nullptr)
+    if (slot) IB3D_SWEEPS(2, true);
+    else if (M == 2) IB3D_SWEEPS(2, false);
+    else IB3D_SWEEPS(1, false);
+#undef IB3D_SWEEPS
 }
 
 // M FP32 sweeps of the right-hand side r (both colours), src -> dst; first:
 // from zero; acc0: first add src to the FP64 unknown
-static void block32(Ctx &c, int M, const float *src, float *dst, const float *r, double omega, bool first,
-                    const double *gate, double *acc0 = nullptr, double *acc1 = nullptr) {
-    const float om = (float)omega, omm = (float)(1.0 - omega);
-    const int64_t NC = c.NC;
-#define IB3D_BLOCK(MM, F, A)                                                                                        \
-    launch_block<float, MM, 24, 8, 8, F, false, A>(c, src, src + NC, dst, dst + NC, r, r + NC, g_axf, g_ayf, g_azf,  \
-                                                   om, omm, gate, 0.5, nullptr, nullptr, acc0, acc1)
+static void launch32(Ctx &c, const SweepPlan &P, int M, const float *src, float *dst, const float *r,
+                     const float *ax, const float *ay, const float *az, double omega, bool first,
+                     const double *gate, double *acc0 = nullptr, double *acc1 = nullptr) {
+    const int64_t NC = P.NC;
+#define IB3D_SWEEPS(MM, F, A)                                                                                       \
+    launch_sweeps<float, MM, F, false, A>(c, P, src, src + NC, dst, dst + NC, r, r + NC, ax, ay, az, (float)omega,   \
+                                          (float)(1.0 - omega), gate, 0.5, nullptr, nullptr, acc0, acc1)
     if (M == 2) {
-        if (first && acc0) IB3D_BLOCK(2, true, true);
-        else if (first) IB3D_BLOCK(2, true, false);
-        else IB3D_BLOCK(2, false, false);
+        if (first && acc0) IB3D_SWEEPS(2, true, true);
+        else if (first) IB3D_SWEEPS(2, true, false);
+        else IB3D_SWEEPS(2, false, false);
     } else {
-        if (first && acc0) IB3D_BLOCK(1, true, true);
-        else if (first) IB3D_BLOCK(1, true, false);
-        else IB3D_BLOCK(1, false, false);
+        if (first && acc0) IB3D_SWEEPS(1, true, true);
+        else if (first) IB3D_SWEEPS(1, true, false);
+        else IB3D_SWEEPS(1, false, false);
     }
-#undef IB3D_BLOCK
+#undef IB3D_SWEEPS
+}
+static void launch32(Ctx &c, const SweepPlan &P, int M, const float *src, float *dst, const float *r, double omega,
+                     bool first, const double *gate, double *acc0 = nullptr, double *acc1 = nullptr) {
+    launch32(c, P, M, src, dst, r, g_axf, g_ayf, g_azf, omega, first, gate, acc0, acc1);
 }
 
-// n >= 2 sweeps as an even number of launches, so that a -> b -> a ends where
-// it began: two sweeps each, then single ones.  calls f(sweeps, launch index).
-template <typename F> static void even_launches(int n, F f) {
-    int two = n / 2, one = n % 2;
-    if ((two + one) % 2) {
-        two--;
-        one += 2;
-    }
-    for (int q = 0; q < two + one; q++) f(q < two ? 2 : 1, q);
-}
-
-// The reference rule on blocks: launches of two sweeps, queued in batches one
-// ahead of the batch the host reads, so the GPU never waits for the host.  The
-// launch in which a sweep falls below epsi stops those after it; if that was
-// its first sweep, it is repeated from its source with one.  Batches are large
-// until the previous solve's count is near, small after: a launch queued after
-// convergence still costs about 3 us.
-static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, double *derr2) {
+// The reference rule with two sweeps per launch, queued in batches one ahead of
+// the batch the host reads, so the GPU never waits for the host.  The launch in
+// which a sweep falls below epsi stops those after it.  If that was its first
+// sweep the launch holds one too many, and the march records only whether a
+// value reached epsi: then the one or two sweeps are repeated from the launch's
+// source.  Batches are large until the previous solve's count is near, small
+// after: a launch queued after convergence still costs about 3 us.
+static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *isum, double *derr2) {
     const double omega = 1.99;
     if (batch_mirror() || second_pc(c)) return -1;
     if (!g_track) IB3D_CHECK(hipMalloc(&g_track, 2 * kRegion * sizeof(double)));
@@ -1753,7 +1731,7 @@ static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, doubl
         IB3D_CHECK(hipMemsetAsync(region, 0, n * kTrackSlots * sizeof(double), c.stream));
         for (int q = 0; q < n; q++) {
             double *slot = region + q * kTrackSlots;
-            block64(c, shape, 2, (int)((queued + q) & 1), omega, nullptr, epsi, prev, slot);
+            launch64(c, P, 2, (int)((queued + q) & 1), omega, nullptr, epsi, prev, slot);
             prev = slot;
         }
         IB3D_CHECK(hipGetLastError());
@@ -1768,7 +1746,7 @@ static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, doubl
         for (int q = 0; q < size[old]; q++, seen++) {
             for (int w = 0; w < 2; w++) {
                 const double *h = g_mirror + old * kRegion + q * kTrackSlots + w * kBlockSub;
-                const double v = *std::max_element(h, h + kBlockSub);
+                double v = *std::max_element(h, h + kBlockSub);
                 const int64_t it = 2 * seen + w + 1;
                 if (it > cap) {
                     set_error("REDBLACKSOR: no convergence within the sweep cap");
@@ -1776,8 +1754,19 @@ static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, doubl
                 }
                 if (v >= epsi) continue;  // the reference loops while derr2 >= epsi
                 const int from = (int)(seen & 1);
-                if (w == 0) block64(c, shape, 1, from, omega, nullptr, 0.0);
-                if (from == 0)   // the result is in the second buffer
+                int at = 1 - from;   // the buffer that holds the result
+                if (P.march()) {
+                    double *p[2] = {from ? g_pc2 : c.pc[0], from ? g_pc2 + c.NC : c.pc[1]};
+                    IB3D_CHECK(hipMemsetAsync(g_track, 0, 2 * sizeof(double), c.stream));
+                    for (int t = 0; t <= w; t++) sweep64_on(c, p, omega, true, g_track + t, nullptr, 0.0);
+                    IB3D_CHECK(hipMemcpyAsync(g_mirror, g_track + w, sizeof(double), hipMemcpyDeviceToHost, c.stream));
+                    IB3D_CHECK(hipStreamSynchronize(c.stream));
+                    v = g_mirror[0];
+                    at = from;
+                } else if (w == 0) {
+                    launch64(c, P, 1, from, omega, nullptr, 0.0);
+                }
+                if (at)
                     for (int col = 0; col < 2; col++)
                         IB3D_CHECK(hipMemcpyAsync(c.pc[col], g_pc2 + col * c.NC, c.NC * sizeof(double),
                                                   hipMemcpyDeviceToDevice, c.stream));
@@ -1796,7 +1785,7 @@ static int reference_blocks(Ctx &c, int shape, double epsi, int64_t *isum, doubl
 // iteration already converged, so the result (and the count) equals the
 // one-iteration-at-a-time loop while the host synchronises once per batch.
 int redblack_sor_reference(Ctx &c, double epsi, int64_t *isum, double *derr2) {
-    if (const int shape = block_shape(c, true)) return reference_blocks(c, shape, epsi, isum, derr2);
+    if (const SweepPlan P = plan64(c); P.kind) return reference_blocks(c, P, epsi, isum, derr2);
     const double omega = 1.99;
     int64_t done = 0;
     int batch = std::max(1, c.batch);
@@ -1886,10 +1875,10 @@ static int sor_l2(Ctx &c, bool mixed, double bn, int64_t *sweeps, int64_t *outer
         IB3D_CHECK(hipGetLastError());
         if (cnn_before_solve(c, c.scalars + 16, c.scalars + 18, resid_rel)) return -1;
     }
-    // temporally blocked launches where they pay and the sweeps of an outer
-    // iteration can end in the buffer they began in
-    const int shape = c.check >= 2 ? block_shape(c, !mixed) : kBlockNone;
-    if (shape && (mixed ? second_e(c) : second_pc(c))) return -1;
+    // launches of two sweeps where an outer iteration holds enough of them
+    const SweepPlan P = mixed ? plan32(c) : plan64(c);
+    const bool two = P.pays(c.check);
+    if (two && (mixed ? second_e(c) : second_pc(c))) return -1;
     residual_async(c, false, mixed, bn, relv, conv, nullptr);
     int64_t o = 0;     // last queued outer iteration
     int64_t seen = 0;  // first index not yet inspected on the host
@@ -1897,22 +1886,21 @@ static int sor_l2(Ctx &c, bool mixed, double bn, int64_t *sweeps, int64_t *outer
         for (int q = 0; q < batch && o < max_outer; q++) {
             o++;
             const double *gate = conv + (o - 1);
-            if (shape && mixed) {
-                even_launches(c.check, [&](int m, int l) {
-                    const bool apply = l == 0 && o > 1;
-                    block32(c, m, l % 2 ? g_e2 : c.e32[0], l % 2 ? c.e32[0] : g_e2, c.r32[0], c.omega, l == 0, gate,
-                            apply ? c.pc[0] : nullptr, apply ? c.pc[1] : nullptr);
-                });
-            } else if (shape) {
-                even_launches(c.check, [&](int m, int l) { block64(c, shape, m, l % 2, c.omega, gate, 0.5); });
-            } else {
-                for (int s = 0; s < c.check; s++) {
-                    if (mixed)
-                        sweep32(c, c.omega, s == 0, s == 0 && o > 1, gate, 0.5);
-                    else
-                        sweep64(c, c.omega, false, nullptr, gate, 0.5);
-                }
+            int s0 = 0;   // sweeps done in place
+            for (; s0 < (two ? P.alone(c.check) : c.check); s0++) {
+                if (mixed)
+                    sweep32(c, c.omega, s0 == 0, s0 == 0 && o > 1, gate, 0.5);
+                else
+                    sweep64(c, c.omega, false, nullptr, gate, 0.5);
             }
+            P.launches(c.check - s0, [&](int m, int l) {
+                const bool first = s0 == 0 && l == 0, apply = first && o > 1;
+                if (mixed)
+                    launch32(c, P, m, l % 2 ? g_e2 : c.e32[0], l % 2 ? c.e32[0] : g_e2, c.r32[0], c.omega, first, gate,
+                             apply ? c.pc[0] : nullptr, apply ? c.pc[1] : nullptr);
+                else
+                    launch64(c, P, m, l % 2, c.omega, gate, 0.5);
+            });
             residual_async(c, mixed, mixed, bn, relv + o, conv + o, gate);
         }
     };
@@ -2809,8 +2797,9 @@ static int g_coarse_tiles = 2;   // first level smoothed by two temporally block
 static int g_fused_restrict = 64;  // levels (from the finest) whose residual is restricted in one pass
 static int g_prolong_pz = 2;       // levels (from the finest) prolonged four cells of a row per thread
 static int g_sweep_tz = 0;        // planes per chunk on the finest level (0: from g_sweep_blocks)
-static int g_sweep_blocks = 480;
-static int g_sweep_blocks_coarse = 192;  // workgroup target below the finest level
+static constexpr int kSweepBlocks = 480, kSweepBlocksCoarse = 192;
+static int g_sweep_blocks = kSweepBlocks;
+static int g_sweep_blocks_coarse = kSweepBlocksCoarse;  // workgroup target below the finest level
 
 static bool sweep2_shape(const MgLevel &L, int &S, int &tz, dim3 &grid) {
     const int64_t plane = L.H * L.sy, smax = 2 * kSweepThreads - 2 * L.H;
@@ -2827,36 +2816,40 @@ static bool sweep2_shape(const MgLevel &L, int &S, int &tz, dim3 &grid) {
     return S + 2 * L.H <= 2 * kSweepThreads;
 }
 
+static void mg_sweeps(Ctx &c, const MgLevel &L, bool finest, int n, bool first, double omega, const double *gate);
 static void mg_smooth(Ctx &c, const MgLevel &L, bool finest, int n, bool first, double omega, const double *gate) {
+    const SorGeom g = level_geom(L);
+    // two sweeps per launch, x -> x2 -> x; on the first g_fused levels unless a
+    // launch shape was asked for, and from level g_coarse_tiles on
+    const bool own_shape = g_sweep_tz > 0 || g_sweep_blocks != kSweepBlocks || g_sweep_blocks_coarse != kSweepBlocksCoarse;
+    if (L.x2 && ((L.level < g_fused && !own_shape) || (g_coarse_tiles > 0 && L.level >= g_coarse_tiles))) {
+        const SweepPlan P = sweep_plan(L.nx, L.ny, L.nz, L.NC, g, false);
+        if (P.pays(n)) {
+            const int alone = P.alone(n);
+            if (alone) mg_sweeps(c, L, finest, alone, first, omega, gate);
+            P.launches(n - alone, [&](int m, int l) {
+                launch32(c, P, m, l % 2 ? L.x2 : L.x, l % 2 ? L.x : L.x2, L.b, L.ax, L.ay, L.az, omega,
+                         first && alone == 0 && l == 0, gate);
+            });
+            return;
+        }
+    }
+    mg_sweeps(c, L, finest, n, first, omega, gate);
+}
+
+// the same by whole sweeps in one launch on the first g_fused levels, else by
+// half-sweeps in place
+static void mg_sweeps(Ctx &c, const MgLevel &L, bool finest, int n, bool first, double omega, const double *gate) {
     const SorGeom g = level_geom(L);
     const float om = (float)omega, omm = (float)(1.0 - omega);
     const dim3 cg(nblocks(L.NC, kSorBlock));
     int S = 0, tz = 0;
     dim3 sg;
-    if (!finest && g_coarse_tiles > 0 && L.level >= g_coarse_tiles && L.x2 && n >= 2 &&
-        (n + 1) / 2 <= kTileMaxSweeps) {
-        // two launches of ceil(n/2) and floor(n/2) sweeps: x -> x2 -> x, on
-        // 8 x 8 x 8 blocks
-        constexpr int T = kTileCube;
-        const dim3 tg((unsigned)((L.sx - 2 + T - 1) / T), (unsigned)((L.sy - 2 + T - 1) / T),
-                      (unsigned)((L.sz - 2 + T - 1) / T));
-        auto launch = [&](int m, bool fz, const float *from, float *to) {
-#define IB3D_TILE(F, MM)                                                                                            \
-    hipLaunchKernelGGL((k_smooth_tile<F, MM, T, T, T>), tg, dim3(kTileThreads), 0, c.stream, from, to, L.b, L.ax,    \
-                       L.ay, L.az, g, om, omm, gate, 0.5)
-            if (m == 2) { if (fz) IB3D_TILE(true, 2); else IB3D_TILE(false, 2); }
-            else { if (fz) IB3D_TILE(true, 1); else IB3D_TILE(false, 1); }
-#undef IB3D_TILE
-        };
-        launch((n + 1) / 2, first, L.x, L.x2);
-        launch(n / 2, false, L.x2, L.x);
-        return;
-    }
     if (L.level < g_fused && L.x2 && n >= 2 && sweep2_shape(L, S, tz, sg)) {
         // an odd count does its first sweep in place, so that the pairs of
         // fused sweeps end in x
         if (n % 2) {
-            mg_smooth(c, L, finest, 1, first, omega, gate);
+            mg_sweeps(c, L, finest, 1, first, omega, gate);
             n -= 1;
             first = false;
         }
@@ -3041,12 +3034,10 @@ static int gmres_cycle(Ctx &c, int m, int k, const double *gate, double target, 
         float *Z = g_kz + j * stride, *Vj = g_kv + j * stride, *Vn = g_kv + (j + 1) * stride;
         if (c.mode == 4) {
             mg_vcycle(c, Vj, Z, aj);
-        } else if (k >= 2 && block_shape(c, false)) {
-            even_launches(k, [&](int mm, int l) {
-                block32(c, mm, l % 2 ? g_e2 : Z, l % 2 ? Z : g_e2, Vj, c.omega, l == 0, aj);
-            });
         } else {
-            for (int sw = 0; sw < k; sw++) {
+            const SweepPlan P = plan32(c);
+            const int alone = P.pays(k) ? P.alone(k) : k;
+            for (int sw = 0; sw < alone; sw++) {
                 for (int col = 0; col < 2; col++) {
                     if (sw == 0)
                         hipLaunchKernelGGL((k_sor_pz<float, false, true, false>), pz_grid(c), tb, 0, c.stream,
@@ -3058,6 +3049,9 @@ static int gmres_cycle(Ctx &c, int m, int k, const double *gate, double target, 
                                            col, om, omm, nullptr, aj, 0.5, nullptr);
                 }
             }
+            P.launches(k - alone, [&](int mm, int l) {
+                launch32(c, P, mm, l % 2 ? g_e2 : Z, l % 2 ? Z : g_e2, Vj, c.omega, alone == 0 && l == 0, aj);
+            });
         }
         hipLaunchKernelGGL(k_matvec32_pz<false>, pz_grid(c), tb, 0, c.stream, Z, Z + NC, V0, V0 + NC, Vn, Vn + NC,
                            g_axf, g_ayf, g_azf, g, aj, 0.5, (const uint32_t *)g_actbits, g_actbits_nw);
@@ -3226,7 +3220,7 @@ static int sor_gmres(Ctx &c, double bn, int64_t *sweeps, int64_t *outer, double 
     if (sor_float_tables(c)) return -1;
     if (gmres_buffers(c, m)) return -1;
     if (c.mode == 4 && mg_setup(c)) return -1;
-    if (c.mode == 3 && k >= 2 && block_shape(c, false) && second_e(c)) return -1;
+    if (c.mode == 3 && plan32(c).pays(k) && second_e(c)) return -1;
     if (clear_for_geometry(c, m)) return -1;
     if (ensure_partial(nblocks(2 * c.NC, kSorBlock))) return -1;
     const int64_t max_outer = std::max<int64_t>(1, c.max_sweeps / ((int64_t)m * k));

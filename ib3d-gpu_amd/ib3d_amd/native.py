@@ -301,15 +301,15 @@ class Solver:
                                       int(max_levels)))
 
     def set_fused_sweeps(self, levels=2, planes=0, blocks=480, coarse_blocks=192):
-        """Multigrid smoothing of the first `levels` levels with one launch
-        per red-black sweep (0: two half-sweep launches everywhere);
-        identical results.  True/False mean 1/0."""
+        """Multigrid smoothing of the first `levels` levels with launches of two
+        red-black sweeps, or of one in the given launch shape (0: two half-sweep
+        launches per sweep everywhere); identical results.  True/False mean 1/0."""
         _ok(self.L.ib3d_set_fused_sweeps(int(levels), int(planes), int(blocks), int(coarse_blocks)))
 
     def set_coarse_tiles(self, from_level=2):
-        """Multigrid levels from `from_level` on (0: none) smoothed by two
-        temporally blocked launches per phase instead of half-sweep
-        launches; identical results.  True/False mean 2/0."""
+        """Multigrid levels from `from_level` on (0: none) smoothed by temporally
+        blocked launches of two sweeps instead of half-sweep launches; identical
+        results.  True/False mean 2/0."""
         if from_level is True:
             from_level = 2
         _ok(self.L.ib3d_set_coarse_tiles(int(from_level)))

@@ -44,9 +44,8 @@ LEVEL1 = None
 # 500-step run, 10.381 / 10.406 at 384x256x256, 29.85 / 29.99 at
 # 512x320x320; 6+6 was better on the last two but not at 256x192x192.
 SMALL = (5, 4)
-# how the smoothing is launched (identical results either way): whole sweeps
-# in one launch on the first `fused` levels, two temporally blocked launches
-# per smoothing phase from level `tiles` on
+# how the smoothing is launched (identical results either way): two sweeps in
+# one launch on the first `fused` levels and from level `tiles` on
 LAUNCH = {"fused": 2, "tiles": 2}
 
 MODES = ("reference", "fp64-cold", "fp64", "mixed-dc", "gmres-sor", "mixed")

@@ -191,19 +191,19 @@ int ib3d_set_multigrid_level(int level, int nu1, int nu2);
  * sweeps cost a barrier each, not a launch, so more of them can pay. */
 int ib3d_set_multigrid_small(int nu1, int nu2);
 /* mode 4: smooth the first `levels` multigrid levels (2, the default: the
- * finest and the next) with whole red-black sweeps in one launch each, the
- * others with two half-sweep launches (0: none), unless they are tiled
- * (ib3d_set_coarse_tiles).  Both give identical results.  planes: z planes
- * per workgroup on the finest level (0: chosen so that the grid holds about
- * `blocks` workgroups); below it the grid holds about `coarse_blocks`
- * (defaults 0, 480 and 192). */
+ * finest and the next) with fused launches, the others with two half-sweep
+ * launches per sweep (0: none), unless they are blocked (ib3d_set_coarse_tiles).
+ * A fused launch does two whole sweeps; with a launch shape given (planes or
+ * other than the default block counts), and for sweeps left over, one.  All give
+ * identical results.  planes: z planes per workgroup on the finest level of the
+ * launches of one sweep (0: chosen so that the grid holds about `blocks`
+ * workgroups); below it the grid holds about `coarse_blocks` (defaults 0, 480
+ * and 192). */
 int ib3d_set_fused_sweeps(int levels, int planes, int blocks, int coarse_blocks);
 /* mode 4: smooth the multigrid levels from `from_level` on (2, the
- * default; 0 for none) that are cycled by launches with two temporally
- * blocked launches per smoothing phase: each workgroup sweeps an 8x8x8 cube
- * plus a halo in LDS, ceil(n/2) sweeps in the first launch and floor(n/2) in
- * the second (n = 2..4), instead of 2n half-sweep launches.  Both give
- * identical results. */
+ * default; 0 for none) that are cycled by launches with temporally blocked
+ * launches of two sweeps instead of half-sweep launches.  Both give identical
+ * results. */
 int ib3d_set_coarse_tiles(int from_level);
 /* mode 4: on the first `levels` multigrid levels (64, the default: every
  * level cycled by launches; 0 for none) form the residual and restrict it to

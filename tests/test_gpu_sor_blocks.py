@@ -1,11 +1,12 @@
-"""Temporally blocked sweeps (k_sor_block) against the oracle's plain loops.
+"""Two sweeps per launch (k_sor_block, k_sor_march) against the oracle's plain
+loops.
 
 FP64: the same operations per cell in the same order, so the iteration count
 and every value of pc must be bit-identical, under the reference rule (whose
 last launch may hold one sweep too many) and in the L2 mode.  FP32 (the defect
 equation): n sweeps from zero differ from n FP64 sweeps by rounding only.  The
-grids lie around the three block shapes' edges and both sides of the size
-rules; one is too large for blocks."""
+grids lie around the block shapes' and the march's tiles' edges and on both sides
+of the size rules."""
 import numpy as np
 import pytest
 
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 # cells per unit length of the uniform box, and the interior grid
 GRIDS = [(4, (32, 24, 24)), (4, (33, 25, 23)), (4, (31, 17, 18)), (6, (42, 40, 39)), (6, (66, 50, 46)),
-         (8, (65, 63, 64)), (8, (73, 66, 57)), (10, (98, 64, 49)), (12, (121, 113, 112))]
+         (8, (65, 63, 64)), (8, (73, 66, 57)), (10, (98, 64, 49)), (12, (121, 113, 112)), (14, (122, 128, 97)),
+         (10, (190, 90, 91)), (12, (119, 93, 73))]
 
 
 def _pair(tmp_path, per, n, scale=1.0, seed=3):
@@ -75,7 +77,7 @@ def test_extreme_values_match_the_oracle(tmp_path, scale):
 
 
 @pytest.mark.parametrize("check", [2, 3, 4, 7, 10])
-@pytest.mark.parametrize("per,n", [GRIDS[1], GRIDS[4], GRIDS[6]])
+@pytest.mark.parametrize("per,n", [GRIDS[1], GRIDS[4], GRIDS[6], GRIDS[8], GRIDS[11]])
 def test_sweep_counts_match_the_oracle(tmp_path, per, n, check):
     """`check` sweeps of the L2 modes: FP64 bitwise, FP32 to rounding."""
     from ib3d_amd.native import IB3DError
