@@ -445,7 +445,7 @@ def main():
             cases.write_case(cfg, case)
             s = Solver.from_case(case)
             s.step()
-            for tiles in (0, 1):
+            for tiles in (4, 1):
                 s.set_momentum_tiles(tiles)
                 for _ in range(3):
                     s.nsMomentum()

@@ -251,6 +251,8 @@ static void free_all(Ctx &c) {
         dfree(c.mrec[t]);
     }
     c.mtn[0] = c.mtn[1] = c.mtn[2] = 0;
+    dfree(c.mom_left);
+    c.mom_rows = 0;
     c.mom_ready = false;
     dfree(c.e32[0]); dfree(c.r32[0]);   // colour 1 lives in the same blocks
     c.e32[1] = nullptr;

@@ -320,9 +320,8 @@ class Solver:
         _ok(self.L.ib3d_set_fused_restrict(int(levels)))
 
     def set_momentum_tiles(self, on=True):
-        """nsMomentum's interior kernel: 0 straight from HBM (the default), 1-3
-        from LDS tiles marching in z, 4 straight from HBM with 64-bit indices;
-        identical results."""
+        """nsMomentum's interior kernel: 0 by size (the default), 1-3 from LDS
+        tiles marching in z, 4 straight from HBM; identical results."""
         _ok(self.L.ib3d_set_momentum_tiles(int(on)))
 
     def set_krylov_target(self, target):

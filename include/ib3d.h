@@ -218,11 +218,10 @@ int ib3d_set_fused_restrict(int levels);
  * correct).  drop_interior != 0 checks the guard without its interior
  * test instead, which reads outside. */
 int ib3d_selfcheck_resid_guard(int64_t nx, int64_t ny, int64_t nz, int drop_interior, int64_t *outside);
-/* nsMomentum's interior columns: on == 0 (the default) reads every stencil
- * value from HBM through 32-bit byte offsets (64-bit indices when the FP64
- * fields span 4 GiB or more); 1, 2, 3 march LDS tiles of 64 x 8, 64 x 4 and
- * 64 x 8 columns (3 and 4 waves per SIMD) in z; 4 reads from HBM with
- * 64-bit indices.  All give identical results. */
+/* nsMomentum's interior columns: on == 0 (the default) chooses by size; 1, 2,
+ * 3 march LDS tiles of 64 x 8 columns in z, with the rows that need a branch in
+ * a second launch; 4 reads every stencil value from HBM.  All give identical
+ * results. */
 int ib3d_set_momentum_tiles(int on);
 /* modes 3 and 4: replay each refinement iteration (Krylov cycle, FP64
  * residual and its norm) as one captured HIP graph (on != 0) or launch its
