@@ -153,7 +153,7 @@ struct TiledFields {
     double m2[3], p2[3];
     int64_t c, sx, sxy;
     template <int f, int a, int b, int d> __device__ __forceinline__ double value() const {
-        static_assert(d >= -1 && d <= 1 || (a == 0 && b == 0), "off the tiles");
+        static_assert((d >= -1 && d <= 1) || (a == 0 && b == 0), "off the tiles");
         if constexpr (d == -2) return m2[f];
         else if constexpr (d == 2) return p2[f];
         else return (d < 0 ? below : d > 0 ? above : here)[f * kTile + a + b * kTileS];
