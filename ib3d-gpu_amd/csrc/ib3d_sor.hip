@@ -2046,11 +2046,11 @@ __device__ __forceinline__ float restrict_at(const MgView &F, const MgView &C, i
                     n++;
                 }
             } else {
-                const float rb = F.b[(int64_t)c * F.NC + f];
-                if (rb == rb) {
-                    s += cell_resid(F, rb, c, f, ii, jj, kk);
-                    n++;
-                }
+                // (of an inactive child NaN: formed all the same, so that the
+                // eight children's reads overlap)
+                const float rb = F.b[(int64_t)c * F.NC + f], v = cell_resid(F, rb, c, f, ii, jj, kk);
+                s = rb == rb ? s + v : s;
+                n += rb == rb ? 1 : 0;
             }
         }
         if (n) out = s / (float)n;
@@ -2313,11 +2313,19 @@ k_mg_prolong_pz(MgView F, MgView C, const uint32_t *__restrict__ bits, int64_t n
 static constexpr int kMgSmallMax = 8;
 static constexpr int kMgSmallThreads = 1024;
 static constexpr int64_t kMgSmallLds = 64 * 1024;
+// division by a level's pairs per row and by its rows
+struct MgDivs {
+    FastDiv half, ny;
+};
 struct MgSmall {
     MgView L[kMgSmallMax];   // global arrays of the levels (x, b used for level 0 only)
     int off[kMgSmallMax];    // LDS offset (floats) of each level's block: x, b (2*NC each), the Laplacian
                              // rows (3*sxp, 3*sy, 3*sz) and, but for the coarsest, the prolongation
                              // tables (sx + sy + sz entries, 16-byte aligned)
+    MgDivs div[kMgSmallMax];
+    const float *image;      // what LDS holds before the cycle
+    int lds;                 // its floats (a multiple of 4); level 0's residual follows if there is room
+    bool room;
     int n, nu1, nu2, ncoarse;
     float om, omc;
 };
@@ -2346,6 +2354,20 @@ __device__ __forceinline__ MgView lds_view(const MgSmall &S, int l, float *lds) 
     }
     return v;
 }
+
+// Who works on a level: the whole workgroup with barriers, or (the smallest
+// levels) its first wave, which needs none between its own LDS accesses.
+struct MgCrew {
+    bool wave;
+    __device__ __forceinline__ int size() const { return wave ? 64 : kMgSmallThreads; }
+    __device__ __forceinline__ void sync() const {
+        asm volatile("" ::: "memory");
+        if (wave)
+            __builtin_amdgcn_wave_barrier();
+        else
+            __syncthreads();
+    }
+};
 
 // one colour half-sweep of red-black SOR over the whole level, then a barrier
 __device__ void blk_sweep(const MgView &L, int c, bool first, float om) {
@@ -2379,209 +2401,228 @@ __device__ void blk_sweep(const MgView &L, int c, bool first, float om) {
     __syncthreads();
 }
 
-// The same sweeps with each thread's share of the level held in registers:
-// a thread owns slots f = tid + 1024 t (t < kMgSlots) of each colour, and
-// what does not change while the level is smoothed (the slot, its
-// right-hand side, the neighbour offset, the six off-diagonal coefficients
-// and the reciprocal of the diagonal) is loaded once per visit of the level
-// instead of once per half-sweep.  The arithmetic is blk_sweep's, operand
-// for operand.
-static constexpr int kMgSlots = 2;   // slots per colour and thread: NC <= 2048 (larger levels: blk_sweep)
-struct MgSlot {
-    int f, s;                        // slot (-1: none or not a cell), ii & 1
-    float rr, a1x, a3x, a1y, a3y, a1z, a3z, rd;  // rd = rcp((a2x + a2y) + a2z)
+// One visit of a level with each thread's share of it in registers: a thread has
+// up to kMgPairs pairs of cells (2m+1, 2m+2) of a row, one of each colour, with
+// their values, right-hand sides and coefficients.  On the way up the coarse
+// correction is added first, then n sweeps, then on the way down the residual
+// is left in r for restrict_pairs.  In a pair one cell's x neighbour is the other,
+// and the outer neighbour of either lies in its own slot of the other colour, so a
+// half-sweep reads five values and writes one; a cell that is not there is computed
+// from the first interior one's neighbours and not stored, so there is no branch
+// and the reads overlap.  The arithmetic is blk_sweep's, prolong_at's and
+// cell_resid's, operand for operand.
+static constexpr int kMgPairs = 2;
+struct MgPair {
+    int s;                        // of the colour-0 cell: ii & 1 (the colour-1 cell: 1 - s)
+    int f[2];                     // slots (-1: no cell)
+    float x[2], rr[2], a1x[2], a3x[2], d[2], rd[2];  // d = (a2x + a2y) + a2z, rd = rcp(d)
+    float a1y, a3y, a1z, a3z;
 };
-__device__ __forceinline__ void blk_cache(const MgView &L, MgSlot (&sl)[2][kMgSlots]) {
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int t = 0; t < kMgSlots; t++) {
-            MgSlot &q = sl[c][t];
-            const int f = (int)threadIdx.x + t * kMgSmallThreads;
-            q.f = -1;
-            if (f >= L.NC) continue;
-            const float rr = L.b[(int64_t)c * L.NC + f];
-            if (!(rr == rr)) continue;
-            int ii, jj, kk;
-            view_decode(L, f, c, ii, jj, kk);
-            q.f = f;
-            q.s = ii & 1;
-            q.rr = rr;
-            q.a1x = L.ax[ii];
-            q.a3x = L.ax[2 * L.sxp + ii];
-            q.a1y = L.ay[jj];
-            q.a3y = L.ay[2 * L.sy + jj];
-            q.a1z = L.az[kk];
-            q.a3z = L.az[2 * L.sz + kk];
-            q.rd = __builtin_amdgcn_rcpf((L.ax[L.sxp + ii] + L.ay[L.sy + jj]) + L.az[L.sz + kk]);
-        }
+__host__ __device__ inline int mg_pairs(const MgView &L) { return ((L.nx + 1) >> 1) * L.ny * L.nz; }
+// pair `id` of a level: cells 2m+1 and 2m+2 of row jj, kk
+__device__ __forceinline__ void pair_decode(const MgView &L, const MgDivs &D, int id, int &m, int &jj, int &kk) {
+    const int row = L.nx <= 2 ? id : (int)fdiv((uint32_t)id, D.half);   // (fdiv takes divisors from 2)
+    m = id - row * ((L.nx + 1) >> 1);
+    const int k = (int)fdiv((uint32_t)row, D.ny);
+    jj = 1 + row - k * L.ny;
+    kk = 1 + k;
 }
-__device__ __forceinline__ void blk_sweep_cached(const MgView &L, const MgSlot (&sl)[kMgSlots], int c, bool first,
-                                                 float om) {
-    float *mine = L.x + (int64_t)c * L.NC;
-    const float *o = L.x + (int64_t)(1 - c) * L.NC;
+template <int T>   // pairs per thread
+__device__ __forceinline__ void sweep_pairs(const MgCrew &W, const MgView &L, MgPair (&pr)[kMgPairs], int n, float om) {
     const int plane = L.H * L.sy;
-    const bool no_other = first && c == 0;
+#pragma unroll 1
+    for (int sweep = 0; sweep < n; sweep++) {
 #pragma unroll
-    for (int t = 0; t < kMgSlots; t++) {
-        const MgSlot &q = sl[t];
-        if (q.f < 0) continue;
-        const int f = q.f;
-        float pw = 0.0f, pe = 0.0f, ps = 0.0f, pn = 0.0f, pb = 0.0f, pt = 0.0f;
-        if (!no_other) {
-            pw = o[f - 1 + q.s];
-            pe = o[f + q.s];
-            ps = o[f - L.H];
-            pn = o[f + L.H];
-            pb = o[f - plane];
-            pt = o[f + plane];
+        for (int c = 0; c < 2; c++) {
+            float *mine = L.x + (int64_t)c * L.NC;
+            const float *o = L.x + (int64_t)(1 - c) * L.NC;
+            float outer[T], ps[T], pn[T], pb[T], pt[T];
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const int f = max(pr[t].f[c], plane + L.H);
+                outer[t] = o[f], ps[t] = o[f - L.H], pn[t] = o[f + L.H], pb[t] = o[f - plane], pt[t] = o[f + plane];
+            }
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                MgPair &q = pr[t];
+                const bool odd = c ? q.s == 0 : q.s == 1;   // ii is odd: the pair's other cell lies east
+                const float pw = odd ? outer[t] : q.x[1 - c], pe = odd ? q.x[1 - c] : outer[t];
+                const float gs = ((((((q.rr[c] - q.a1x[c] * pw) - q.a3x[c] * pe) - q.a1y * ps[t]) - q.a3y * pn[t]) -
+                                   q.a1z * pb[t]) - q.a3z * pt[t]) * q.rd[c];
+                const float x = (1.0f - om) * q.x[c] + om * gs;
+                if (q.f[c] >= 0 && q.rr[c] == q.rr[c]) {
+                    q.x[c] = x;
+                    mine[q.f[c]] = x;
+                }
+            }
+            W.sync();
         }
-        const float pold = first ? 0.0f : mine[f];
-        const float gs =
-            ((((((q.rr - q.a1x * pw) - q.a3x * pe) - q.a1y * ps) - q.a3y * pn) - q.a1z * pb) - q.a3z * pt) * q.rd;
-        mine[f] = (1.0f - om) * pold + om * gs;
     }
-    __syncthreads();
+}
+__device__ __forceinline__ void visit_pairs(const MgCrew &W, const MgView &L, const MgView &C, const MgDivs &D, int n,
+                                            bool down, float om, float *r) {
+    MgPair pr[kMgPairs];
+    const int pairs = mg_pairs(L), plane = L.H * L.sy;
+#pragma unroll
+    for (int t = 0; t < kMgPairs; t++) {
+        MgPair &q = pr[t];
+        q = MgPair{};
+        q.f[0] = q.f[1] = -1;
+        const int id = (int)threadIdx.x + t * W.size();
+        if (id >= pairs) continue;
+        int m, jj, kk;
+        pair_decode(L, D, id, m, jj, kk);
+        q.s = (jj + kk) & 1 ? 1 : 0;   // 2m+1 is of colour 0 where jj + kk is odd
+        q.a1y = L.ay[jj];
+        q.a3y = L.ay[2 * L.sy + jj];
+        q.a1z = L.az[kk];
+        q.a3z = L.az[2 * L.sz + kk];
+        const float d2 = L.ay[L.sy + jj], d3 = L.az[L.sz + kk];
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int ii = 2 * m + 1 + (c ? q.s : 1 - q.s);
+            const int f = (ii >> 1) + L.H * (jj + L.sy * kk);
+            if (ii > L.nx) continue;
+            q.f[c] = f;
+            q.rr[c] = L.b[(int64_t)c * L.NC + f];
+            q.a1x[c] = L.ax[ii];
+            q.a3x[c] = L.ax[2 * L.sxp + ii];
+            q.d[c] = (L.ax[L.sxp + ii] + d2) + d3;
+            q.rd[c] = __builtin_amdgcn_rcpf(q.d[c]);
+            if (!down && q.rr[c] == q.rr[c]) {
+                q.x[c] = L.x[(int64_t)c * L.NC + f] + prolong_at(L, C, ii, jj, kk);
+                L.x[(int64_t)c * L.NC + f] = q.x[c];
+            }
+        }
+    }
+    if (!down) W.sync();
+    if (pairs <= W.size())
+        sweep_pairs<1>(W, L, pr, n, om);
+    else
+        sweep_pairs<2>(W, L, pr, n, om);
+    if (!r) return;
+#pragma unroll
+    for (int t = 0; t < kMgPairs; t++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const MgPair &q = pr[t];
+            if (q.f[c] < 0) continue;
+            const int f = q.f[c];
+            const float *o = L.x + (int64_t)(1 - c) * L.NC;
+            const bool odd = c ? q.s == 0 : q.s == 1;
+            const float outer = o[f], pw = odd ? outer : q.x[1 - c], pe = odd ? q.x[1 - c] : outer;
+            const float ax = (((((q.a1x[c] * pw + q.a3x[c] * pe) + q.a1y * o[f - L.H]) + q.a3y * o[f + L.H]) +
+                               q.a1z * o[f - plane]) + q.a3z * o[f + plane]) + q.d[c] * q.x[c];
+            r[c * L.NC + f] = q.rr[c] - ax;   // (NaN at a cell that is not solved for)
+        }
+    W.sync();
+}
+// restrict_at on every coarse cell, from the residuals in r
+__device__ __forceinline__ void restrict_pairs(const MgCrew &W, const MgView &F, const MgView &C, const MgDivs &D,
+                                               const float *r) {
+    const int pairs = mg_pairs(C);
+    for (int id = (int)threadIdx.x; id < pairs; id += W.size()) {
+        int m, J, K;
+        pair_decode(C, D, id, m, J, K);
+#pragma unroll 1
+        for (int I = 2 * m + 1; I <= min(2 * m + 2, C.nx); I++) {
+            float v[8], s = 0.0f;
+            int n = 0;
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const int ii = 2 * I - 1 + (t & 1), jj = 2 * J - 1 + ((t >> 1) & 1), kk = 2 * K - 1 + (t >> 2);
+                v[t] = r[((ii + jj + kk) & 1) * F.NC + (jj + F.sy * kk) * F.H + (ii >> 1)];
+            }
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                s = v[t] == v[t] ? s + v[t] : s;
+                n += v[t] == v[t] ? 1 : 0;
+            }
+            C.b[(int64_t)((I + J + K) & 1) * C.NC + (J + C.sy * K) * C.H + (I >> 1)] = n ? s / (float)n : __builtin_nanf("");
+        }
+    }
+    W.sync();
 }
 
-__device__ void blk_resid_restrict(const MgView &F, const MgView &C) {
-    for (int q = threadIdx.x; q < 2 * C.NC; q += blockDim.x) {
+__device__ __forceinline__ void blk_resid_restrict(const MgCrew &W, const MgView &F, const MgView &C) {
+    for (int q = threadIdx.x; q < 2 * C.NC; q += W.size()) {
         const int cc = q >= C.NC ? 1 : 0;
         const int fc = q - cc * C.NC;
         int I, J, K;
         view_decode(C, fc, cc, I, J, K);
         C.b[q] = restrict_at<false>(F, C, cc, fc, I, J, K);
     }
-    __syncthreads();
+    W.sync();
 }
 
-__device__ void blk_prolong(const MgView &F, const MgView &C) {
-    for (int q = threadIdx.x; q < 2 * F.NC; q += blockDim.x) {
+__device__ __forceinline__ void blk_prolong(const MgCrew &W, const MgView &F, const MgView &C) {
+    for (int q = threadIdx.x; q < 2 * F.NC; q += W.size()) {
         if (!(F.b[q] == F.b[q])) continue;
         const int c = q >= F.NC ? 1 : 0;
         int ii, jj, kk;
         view_decode(F, q - c * F.NC, c, ii, jj, kk);
         F.x[q] += prolong_at(F, C, ii, jj, kk);
     }
-    __syncthreads();
-}
-
-// The constant tables of a level as one run of 32-bit words: the Laplacian
-// rows (3 x sxp, 3 x sy, 3 x sz) and, with `tables`, the prolongation tables
-// (4 words per entry: nx+2, sy, sz entries).  Word q's global source and LDS
-// destination (false past the end).
-static constexpr int kMgGather = 8;
-__device__ __forceinline__ int mg_table_words(const MgView &G, bool tables) {
-    return 3 * (G.sxp + G.sy + G.sz) + (tables ? 4 * (G.nx + 2 + G.sy + G.sz) : 0);
-}
-__device__ __forceinline__ bool mg_table_word(const MgView &G, const MgView &V, bool tables, int q, const float *&src,
-                                              float *&dst) {
-    const int r = 3 * (G.sxp + G.sy + G.sz);
-    if (q < r) {
-        // the three row tables are contiguous in LDS (lds_view) and each is
-        // its own global array
-        const int ay = 3 * G.sxp, az = ay + 3 * G.sy;
-        src = q < ay ? G.ax + q : q < az ? G.ay + (q - ay) : G.az + (q - az);
-        dst = const_cast<float *>(V.ax) + q;
-        return true;
-    }
-    if (!tables) return false;
-    q -= r;
-    const int ty = 4 * (G.nx + 2), tz = ty + 4 * G.sy;
-    if (q >= tz + 4 * G.sz) return false;
-    src = q < ty ? reinterpret_cast<const float *>(G.tx) + q
-                 : q < tz ? reinterpret_cast<const float *>(G.ty) + (q - ty) : reinterpret_cast<const float *>(G.tz) + (q - tz);
-    dst = reinterpret_cast<float *>(const_cast<MgAxis *>(V.tx)) + q;
-    return true;
+    W.sync();
 }
 
 // V-cycle over levels S.L[0..n): x of level 0 from its b.  x and b of every
 // level live in dynamic LDS for the duration (2 x 2*NC floats per level);
 // S.L[0]'s global b is read at the start and its global x written at the end.
+// Latency from end to end, on one compute unit whose instruction cache is cold:
+// so one copy of each piece of code, few instructions, and no barrier where a
+// wave suffices.  From 16x8x8 down with 5+4 sweeps (44 half-sweeps) 18 us, from
+// 16x12x12 27; 29 and 36 with the tables gathered word by word (9 us), a
+// workgroup barrier per half-sweep on every level, and a thread per padded slot.
 __global__ void __launch_bounds__(kMgSmallThreads) k_mg_small(MgSmall S, const double *gate, double thr) {
     if (gated(gate, thr)) return;
-    extern __shared__ float lds[];
-    // Everything the cycle reads from global memory (level 0's b, every
-    // level's Laplacian rows and prolongation tables) is gathered in passes
-    // in which each thread issues all of its loads before it stores any, so
-    // one pass costs one memory latency: x is zeroed (cells outside the
-    // solve hold 0) while the loads are in flight.
-    const int tid = (int)threadIdx.x, nt = (int)blockDim.x;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    // The whole of LDS as mg_setup has laid it out (x = 0, each level's tables),
+    // level 0's b from its own array, in wide copies that are all in flight at
+    // once.
+    const int tid = (int)threadIdx.x;
     {
-        const MgView V = lds_view(S, 0, lds), G = S.L[0];
-        for (int q0 = 0; q0 < 2 * V.NC; q0 += kMgGather * nt) {
-            float v[kMgGather];
+        const float4 *img = reinterpret_cast<const float4 *>(S.image), *b0 = reinterpret_cast<const float4 *>(S.L[0].b);
+        const int q0 = S.off[0] / 4 + S.L[0].NC / 2, q1 = q0 + S.L[0].NC / 2;   // level 0's b in LDS
+        float4 v[kMgSmallLds / (16 * kMgSmallThreads)];
 #pragma unroll
-            for (int t = 0; t < kMgGather; t++) {
-                const int q = min(q0 + tid + t * nt, 2 * V.NC - 1);
-                v[t] = G.b[q];
-            }
-#pragma unroll
-            for (int t = 0; t < kMgGather; t++) {
-                const int q = q0 + tid + t * nt;
-                if (q < 2 * V.NC) V.b[q] = v[t];
-            }
-        }
-    }
-    for (int l = 0; l < S.n; l++) {
-        const MgView V = lds_view(S, l, lds);
-        for (int q = tid; q < 2 * V.NC; q += nt) V.x[q] = 0.0f;
-    }
-    int words = 0;
-    for (int l = 0; l < S.n; l++) words += mg_table_words(S.L[l], l + 1 < S.n);
-    for (int w0 = 0; w0 < words; w0 += kMgGather * nt) {
-        float v[kMgGather];
-        const float *a[kMgGather];
-        float *d[kMgGather];
-        // word w of the levels' tables in order (clamped to the last): its
-        // source and destination first, then all the loads, then the stores
-#pragma unroll
-        for (int t = 0; t < kMgGather; t++) {
-            const int w = min(w0 + tid + t * nt, words - 1);
-            a[t] = S.L[0].ax;
-            d[t] = nullptr;
-            for (int l = 0, base = 0; l < S.n; l++) {
-                const int n = mg_table_words(S.L[l], l + 1 < S.n);
-                if (w >= base && w < base + n)
-                    mg_table_word(S.L[l], lds_view(S, l, lds), l + 1 < S.n, w - base, a[t], d[t]);
-                base += n;
-            }
+        for (int t = 0; t < (int)(sizeof v / sizeof v[0]); t++) {
+            const int q = tid + t * kMgSmallThreads;
+            if (q < S.lds / 4) v[t] = q >= q0 && q < q1 ? b0[q - q0] : img[q];
         }
 #pragma unroll
-        for (int t = 0; t < kMgGather; t++) v[t] = *a[t];
-#pragma unroll
-        for (int t = 0; t < kMgGather; t++)
-            if (w0 + tid + t * nt < words) *d[t] = v[t];
+        for (int t = 0; t < (int)(sizeof v / sizeof v[0]); t++) {
+            const int q = tid + t * kMgSmallThreads;
+            if (q < S.lds / 4) reinterpret_cast<float4 *>(lds)[q] = v[t];
+        }
     }
     __syncthreads();
-    // n sweeps on level L (the first from zero when `first`), from registers
-    // when the level's slots fit kMgSlots per thread
-    MgSlot sl[2][kMgSlots];
-    auto smooth = [&](const MgView &L, int n, bool first, float om) {
-        if (L.NC <= kMgSlots * kMgSmallThreads) {
-            blk_cache(L, sl);
-            for (int s = 0; s < n; s++) {
-                blk_sweep_cached(L, sl[0], 0, first && s == 0, om);
-                blk_sweep_cached(L, sl[1], 1, first && s == 0, om);
-            }
+    // down to the coarsest level and up again, each piece of code once (three
+    // inlined copies of the sweeps cost 10 us a cycle)
+    MgCrew W{false};
+#pragma unroll 1
+    for (int i = 0; i < 2 * S.n - 1; i++) {
+        const bool down = i < S.n, last = i == S.n - 1;
+        const int l = down ? i : 2 * S.n - 2 - i;
+        const MgView F = lds_view(S, l, lds), C = lds_view(S, min(l + 1, S.n - 1), lds);
+        const bool was = W.wave;
+        W.wave = mg_pairs(F) <= kMgPairs * 64;
+        if (was && !W.wave) __syncthreads();
+        if (W.wave && tid >= 64) continue;
+        const int n = last ? S.ncoarse : down ? S.nu1 : S.nu2;
+        const float om = last ? S.omc : S.om;
+        const bool small = mg_pairs(F) <= kMgPairs * kMgSmallThreads;
+        float *r = small && S.room && down && !last ? lds + S.lds : nullptr;
+        if (small) {
+            visit_pairs(W, F, C, S.div[l], n, down, om, r);
         } else {
-            for (int s = 0; s < n; s++) {
-                blk_sweep(L, 0, first && s == 0, om);
-                blk_sweep(L, 1, first && s == 0, om);
-            }
+            if (!down) blk_prolong(W, F, C);
+            for (int q = 0; q < 2 * n; q++) blk_sweep(F, q & 1, down && q < 2, om);
         }
-    };
-    for (int l = 0; l + 1 < S.n; l++) {
-        const MgView F = lds_view(S, l, lds);
-        smooth(F, S.nu1, true, S.om);
-        blk_resid_restrict(F, lds_view(S, l + 1, lds));
+        if (r) restrict_pairs(W, F, C, S.div[l + 1], r);
+        else if (down && !last) blk_resid_restrict(W, F, C);
     }
-    smooth(lds_view(S, S.n - 1, lds), S.ncoarse, true, S.omc);
-    for (int l = S.n - 2; l >= 0; l--) {
-        const MgView F = lds_view(S, l, lds);
-        blk_prolong(F, lds_view(S, l + 1, lds));
-        smooth(F, S.nu2, false, S.om);
-    }
+    __syncthreads();
     const MgView V0 = lds_view(S, 0, lds);
     for (int q = threadIdx.x; q < 2 * V0.NC; q += blockDim.x) S.L[0].x[q] = V0.x[q];
 }
@@ -2599,6 +2640,7 @@ struct MgLevel {
 static std::vector<MgLevel> g_mg;
 static int g_mg_small = 0;  // first level cycled inside the single-workgroup kernel (= size: none)
 static int g_mg_lds = 0;    // its dynamic LDS bytes
+static float *g_mg_image = nullptr;   // and what they hold before a cycle
 static int64_t g_mg_key[4] = {0, 0, 0, 0};
 
 static SorGeom level_geom(const MgLevel &L) {
@@ -2623,6 +2665,8 @@ void mg_release() {
         if (L.r) (void)hipFree(L.r);
         if (L.x2) (void)hipFree(L.x2);
     }
+    if (g_mg_image) (void)hipFree(g_mg_image);
+    g_mg_image = nullptr;
     g_mg.clear();
     g_mg_key[0] = g_mg_key[1] = g_mg_key[2] = g_mg_key[3] = 0;
 }
@@ -2754,8 +2798,11 @@ static int mg_setup(Ctx &c) {
         bytes += b;
     }
     g_mg_lds = (int)bytes;
+    std::vector<float> image(bytes / 4, 0.0f);
+    size_t at = 0;   // of the level's block in it
     for (int l = 0; l < nl; l++) {
         MgLevel &L = g_mg[l];
+        const size_t rows_at = at + 4 * L.NC, tables_at = rows_at + ((3 * (L.sxp + L.sy + L.sz) + 3) & ~int64_t(3));
         if (check_fastdiv((int)L.H, L.NC + 1) || check_fastdiv((int)L.sy, L.NC / L.H + 1)) {
             set_error("poissonSolver: fast division self-check failed on a multigrid level");
             return -1;
@@ -2777,11 +2824,23 @@ static int mg_setup(Ctx &c) {
             IB3D_CHECK(h2d(L.tx, tx.data(), tx.size() * sizeof(MgAxis)));
             IB3D_CHECK(h2d(L.ty, ty.data(), ty.size() * sizeof(MgAxis)));
             IB3D_CHECK(h2d(L.tz, tz.data(), tz.size() * sizeof(MgAxis)));
+            if (l >= g_mg_small) {
+                MgAxis *t = reinterpret_cast<MgAxis *>(&image[tables_at]);
+                std::copy_n(tx.begin(), L.sx, t);
+                std::copy_n(ty.begin(), L.sy, t + L.sx);
+                std::copy_n(tz.begin(), L.sz, t + L.sx + L.sy);
+            }
         }
         if (l == 0) continue;
         const std::vector<float> rx = mg_rows(mg_faces(c.hx1, c.nx, l), true, L.sxp);
         const std::vector<float> ry = mg_rows(mg_faces(c.hy1, c.ny, l), false, L.sy);
         const std::vector<float> rz = mg_rows(mg_faces(c.hz1, c.nz, l), false, L.sz);
+        if (l >= g_mg_small) {
+            std::copy(rx.begin(), rx.end(), image.begin() + rows_at);
+            std::copy(ry.begin(), ry.end(), image.begin() + rows_at + rx.size());
+            std::copy(rz.begin(), rz.end(), image.begin() + rows_at + rx.size() + ry.size());
+            at += mg_lds_floats((int)L.NC, (int)L.sx, (int)L.sy, (int)L.sz, (int)L.sxp, l < nl - 1);
+        }
         IB3D_CHECK(hipMalloc(&L.ax, rx.size() * 4));
         IB3D_CHECK(hipMalloc(&L.ay, ry.size() * 4));
         IB3D_CHECK(hipMalloc(&L.az, rz.size() * 4));
@@ -2795,6 +2854,10 @@ static int mg_setup(Ctx &c) {
         IB3D_CHECK(dzero(L.x, 2 * L.NC * sizeof(float)));   // cells outside the solve stay 0
         hipLaunchKernelGGL(k_fill_nan_f32, dim3(nblocks(2 * L.NC, kSorBlock)), dim3(kSorBlock), 0, c.stream,
                            L.b, 2 * L.NC);
+    }
+    if (!image.empty()) {
+        IB3D_CHECK(hipMalloc(&g_mg_image, image.size() * sizeof(float)));
+        IB3D_CHECK(h2d(g_mg_image, image.data(), image.size() * sizeof(float)));
     }
     // the fused sweeps' second buffer on every level smoothed by launches:
     // cells they never write (walls, and whatever lies outside the solve)
@@ -2968,16 +3031,22 @@ static void mg_vcycle(Ctx &c, const float *v, float *z, const double *gate) {
         S.nu1 = c.mg_nu_small[0] >= 0 ? c.mg_nu_small[0] : c.mg_nu1c;
         S.nu2 = c.mg_nu_small[1] >= 0 ? c.mg_nu_small[1] : c.mg_nu2c;
         S.ncoarse = c.mg_coarse;
+        S.image = g_mg_image;
+        S.lds = g_mg_lds / 4;
+        const int64_t bytes = g_mg_lds + 8 * g_mg[ns].NC;   // with the residual
+        S.room = bytes <= kMgSmallLds;
         S.om = (float)c.mg_omega;
         S.omc = (float)c.mg_coarse_omega;
         int off = 0;
         for (int l = ns; l < nl; l++) {
             const MgLevel &L = g_mg[l];
             S.L[l - ns] = level_view(L);
+            S.div[l - ns] = {make_fastdiv((int)((L.nx + 1) / 2)), make_fastdiv((int)L.ny)};
             S.off[l - ns] = off;
             off += mg_lds_floats((int)L.NC, (int)L.sx, (int)L.sy, (int)L.sz, (int)L.sxp, l < nl - 1);
         }
-        hipLaunchKernelGGL(k_mg_small, dim3(1), dim3(kMgSmallThreads), g_mg_lds, c.stream, S, gate, 0.5);
+        hipLaunchKernelGGL(k_mg_small, dim3(1), dim3(kMgSmallThreads), S.room ? (int)bytes : g_mg_lds, c.stream, S,
+                           gate, 0.5);
     } else {
         mg_smooth(c, g_mg[nl - 1], false, c.mg_coarse, true, c.mg_coarse_omega, gate);
     }
@@ -3215,6 +3284,7 @@ static int cycle_graph(Ctx &c, int m, int k, double *relv, double *conv) {
     key.push_back((uint64_t)c.mg_coarse);
     key.push_back((uint64_t)g_mg_small);
     key.push_back((uint64_t)g_mg_lds);
+    P(g_mg_image);
     D(c.omega);
     D(c.tol);
     D(c.mg_omega);
