@@ -29,14 +29,19 @@
 // out of its range is asked once per chunk, which is then marched again with
 // divisions.
 //
+// The first eight planes of a chunk only feed the ones above them, by one more
+// update every two planes, so their steps do none to three of the four: 20 of the
+// 160 updates per slot of a chunk of 32 planes (FP64 with TRACK 38.0 -> 35.4 us per
+// sweep at 256x192x192, FP32 17.3 -> 16.5).
+//
 // What bounds it: vector arithmetic (55-60% of the issue slots; the rest is the
 // four updates' chain, 15 LDS reads per step and the barrier, at four waves per
-// SIMD), of which the halo is 1.8 times at 256x192x192.  us per sweep, k_sor_pz
-// (FP32: k_sweep2_pz) -> here: FP64 48.7 -> 40.2 at 256x192x192, with TRACK 66.8
-// -> 44.0; 180 -> 98.9 with TRACK at 384x256x256 (the half-sweeps' atomicMax and,
-// from 384x256x256 on, an Infinity Cache that no longer holds the arrays); FP32
-// 25-28 -> 18.6 at 256x192x192, 63.7 -> 46.8 at 384x256x256 (half-sweeps), level 1
-// of 256x192x192 (128x96x96) 9.2 -> 7.2.
+// SIMD), of which the halo is 1.65 times at 256x192x192.  us per sweep, k_sor_pz
+// (FP32: k_sweep2_pz) -> here: FP64 with TRACK 66.8 -> 35.4 at 256x192x192, 180 ->
+// 92 at 384x256x256 (the half-sweeps' atomicMax and, from 384x256x256 on, an
+// Infinity Cache that no longer holds the arrays); FP32 25-28 -> 16.5 at
+// 256x192x192, 63.7 -> 43.3 at 384x256x256 (half-sweeps), level 1 of 256x192x192
+// (128x96x96) 9.2 -> 6.1.
 //
 // Measured and dropped: one step at a time with every update in a branch of its
 // own (FP64 48 us per sweep, FP32 28.5); the four updates together but the rings
@@ -160,9 +165,9 @@ k_sor_march(const T *__restrict__ s0, const T *__restrict__ s1, T *__restrict__ 
             o2 = o1;
             o1 = o0;
         };
-        // ph = (k - ka) mod 12
-        auto step = [&](auto phc, int k) {
-            constexpr int ph = decltype(phc)::value, q = (q0 + ph) & 1;
+        // ph = (k - ka) mod 12; the first U of the four updates
+        auto step = [&](auto phc, auto uc, int k) {
+            constexpr int ph = decltype(phc)::value, q = (q0 + ph) & 1, U = decltype(uc)::value;
             // ring entries of planes k .. k-5, with plane k at entry ph mod 3
             constexpr int e0 = ph % 3, e1 = (ph + 2) % 3, e2 = (ph + 1) % 3, e3 = e0, e4 = e1, e5 = e2;
             constexpr int f1 = (ph + 3) % 4, f2 = (ph + 2) % 4, f3 = (ph + 1) % 4, f4 = ph % 4;
@@ -204,12 +209,15 @@ k_sor_march(const T *__restrict__ s0, const T *__restrict__ s1, T *__restrict__ 
                 const T pnew = omm * pold + omega * (F ? block_div(v, den, block_rcp(den)) : sor_div(v, den));
                 return live ? pnew : pold;
             };
-            const T g1 = part(0, rhs1, bo1, bo2, za[f1]), g2 = part(1, rhs2, ra2, old1, za[f2]),
-                    g3 = part(2, rhs3, ba3, ba4, za[f3]), g4 = part(3, rhs4, rc4, rc5, za[f4]);
-            const T v1 = relax(g1, n.bo, zc[f1], zd[f1], ro, live1);
-            const T v2 = relax(g2, v1, zc[f2], zd[f2], bo2, live2);
-            const T v3 = relax(g3, v2, zc[f3], zd[f3], old1, live3);
-            const T v4 = relax(g4, v3, zc[f4], zd[f4], ba4, live4);
+            T g1 = 0, g2 = 0, g3 = 0, g4 = 0, v1 = ro, v2 = bo2, v3 = old1, v4 = ba4;
+            if (U > 0) g1 = part(0, rhs1, bo1, bo2, za[f1]);
+            if (U > 1) g2 = part(1, rhs2, ra2, old1, za[f2]);
+            if (U > 2) g3 = part(2, rhs3, ba3, ba4, za[f3]);
+            if (U > 3) g4 = part(3, rhs4, rc4, rc5, za[f4]);
+            if (U > 0) v1 = relax(g1, n.bo, zc[f1], zd[f1], ro, live1);
+            if (U > 1) v2 = relax(g2, v1, zc[f2], zd[f2], bo2, live2);
+            if (U > 2) v3 = relax(g3, v2, zc[f3], zd[f3], old1, live3);
+            if (U > 3) v4 = relax(g4, v3, zc[f4], zd[f4], ba4, live4);
             if (TRACK) {
                 if (k - 1 >= k0 && k - 1 < k1) hot[0] |= (double)fabs(v1 - ro) >= thr;
                 if (k - 2 >= k0 && k - 2 < k1) hot[0] |= (double)fabs(v2 - bo2) >= thr;
@@ -238,12 +246,18 @@ k_sor_march(const T *__restrict__ s0, const T *__restrict__ s1, T *__restrict__ 
         };
 #pragma unroll
         for (int q = 0; q <= AHEAD; q++) load(ka + q, in_[q]);
-        for (int k = ka; k <= kb; k += 12) {
+        // the first planes only feed the updates above them: plane k0 - 3 is the
+        // first to need one update, k0 - 2 two, k0 - 1 three, k0 four
+#define IB3D_STEP(P, U) step(std::integral_constant<int, P>{}, std::integral_constant<int, U>{}, ka + P);
+        IB3D_STEP(0, 0) IB3D_STEP(1, 0) IB3D_STEP(2, 1) IB3D_STEP(3, 1) IB3D_STEP(4, 2) IB3D_STEP(5, 2) IB3D_STEP(6, 3)
+        IB3D_STEP(7, 3)
+#undef IB3D_STEP
+        for (int k = ka; k + 8 <= kb; k += 12) {
 #define IB3D_STEP(P)                                                                                                \
     if (k + P > kb) break;                                                                                          \
-    step(std::integral_constant<int, P>{}, k + P);
-            IB3D_STEP(0) IB3D_STEP(1) IB3D_STEP(2) IB3D_STEP(3) IB3D_STEP(4) IB3D_STEP(5)
-            IB3D_STEP(6) IB3D_STEP(7) IB3D_STEP(8) IB3D_STEP(9) IB3D_STEP(10) IB3D_STEP(11)
+    step(std::integral_constant<int, P % 12>{}, std::integral_constant<int, 4>{}, k + P);
+            IB3D_STEP(8) IB3D_STEP(9) IB3D_STEP(10) IB3D_STEP(11) IB3D_STEP(12) IB3D_STEP(13) IB3D_STEP(14)
+            IB3D_STEP(15) IB3D_STEP(16) IB3D_STEP(17) IB3D_STEP(18) IB3D_STEP(19)
 #undef IB3D_STEP
         }
         return F && range.unsafe();
