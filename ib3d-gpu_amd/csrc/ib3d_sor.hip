@@ -1526,13 +1526,18 @@ static int second_e(Ctx &c) {
 //   18k cells  14.9 |  3.5 |  4.3 |  6.5 |           49k  17.6 |  4.1 |  4.4 |  6.5 |
 //   147k       17.8 |  6.3 |  6.0 |  6.9 |           301k 18.7 | 10.0 |  7.7 |  7.5 |
 //   524k       16.5 | 14.9 | 11.2 |  8.2 | 11.4      1.47M 20.1 |     | 22.3 | 15.1 | 16.8
-//   1.70M      21.3 |      | 27.5 | 20.9 | 17.9      9.4M  66.8 |     |      |      | 44.0
-//   25M       180.0 |      |      |      | 98.9
+//   1.70M      21.3 |      | 27.5 | 20.9 | 17.9      9.4M  66.8 |     |      |      | 35.4
+//   25M       180.0 |      |      |      | 87.2
 // and per FP32 sweep, half-sweep launches | 8x8x4 | 24x8x8 | march:
 //   18k  11.7 | 2.6 |  3.1 |        66k  16.1 | 2.8 |  3.2 |  5.0     147k 14.9 | 3.6 | 3.4 | 5.1
 //   524k 12.7 | 6.8 |  4.8 |  6.0   819k 16.5 |     |  6.7 |  6.7     1.2M 16.5 |    | 8.1 | 7.2
-//   1.7M 15.4 |     |  9.9 |  7.8   3.1M 15.9 |     | 14.4 | 10.0     9.4M 29.0 |  | 38.4 | 18.6
-//   25M  63.7 |     |      | 46.8   52M  181  |     |      | 83.8
+//   1.7M 15.4 |     |  9.9 |  7.8   3.1M 15.9 |     | 14.4 | 10.0     9.4M 29.0 |  | 38.4 | 16.5
+//   25M  63.7 |     |      | 43.3   52M  181  |     |      | 83.8
+// The line between the largest blocks and the march is where the blocks no longer
+// run at once (one per CU in FP64, two in FP32); a sweep of a whole solve, blocks /
+// march, on either side of it: FP64 128x80x64 (240 blocks) 8.6 / 10.4, 128x96x64
+// (288) 13.7 / 11.0, 144x100x96 14.7 / 12.9; FP32 128x80x64 (480) 6.2 / 6.3,
+// 128x96x64 (576) 7.7 / 7.2.
 enum SweepKind { kPlanNone = 0, kBlock884, kBlock888, kBlock24168, kBlock2488, kMarch3628, kMarch3232 };
 struct SweepPlan {
     SweepKind kind = kPlanNone;
@@ -1574,7 +1579,8 @@ static SweepPlan sweep_plan(int64_t nx, int64_t ny, int64_t nz, int64_t NC, cons
     if (NC >= (int64_t)1 << 28) return P;   // 32-bit byte offsets into a colour array
     P.NC = NC;
     P.g = g;
-    if (cells > (fp64 ? 1500000 : 800000)) {
+    const int64_t largest = ((nx + 23) / 24) * ((ny + (fp64 ? 15 : 7)) / (fp64 ? 16 : 8)) * ((nz + 7) / 8);
+    if (cells > (fp64 ? 262144 : 65536) && largest > (fp64 ? 256 : 512)) {
         // one workgroup per CU: the chunk count with the fewest steps (a chunk of
         // tz planes marches tz + 8), over both tile shapes
         const int shape[2][2] = {{32, 32}, {36, 28}};
