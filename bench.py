@@ -39,8 +39,8 @@ the learned form's measurement beside it.  After the timed steps, the
 configuration's whole stated run (500 steps, t = 1.0) of the headline mode
 and of the learned form is timed on its own (`full_run`).
 
-Roofline: the dominant kernel of mode 4 is the finest multigrid level's
-FP32 red-black sweep in one launch (k_sweep2_pz); algorithmic bytes per
+Roofline: for mode 4 the finest multigrid level's FP32 red-black sweep in one
+launch (k_sweep2_pz; the solver does two per launch); algorithmic bytes per
 launch = 12 B per interior cell (old value and right-hand side read, new
 value written, both colours).  For the SOR modes it is the half-sweep:
 16 B (FP64) or 8 B (FP32) per interior cell per launch.  The average launch
@@ -491,7 +491,7 @@ def main():
         main_fields = {f: s.download(f) for f in ("u", "p")}
         log(f"[bench] {a.mode}: {main_res}")
         prec = 32 if a.mode.startswith("mixed") or a.mode == "gmres-sor" else 64
-        # the dominant kernel: the finest level's whole FP32 sweep in mode 4,
+        # the smoother's sweep: the finest level's whole FP32 sweep in mode 4,
         # the half-sweep otherwise
         rprec = 33 if a.mode.startswith("mixed") else prec
         roof = kernel_roofline(s, rprec, a.omega, n_cells)

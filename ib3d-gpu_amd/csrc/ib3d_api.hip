@@ -109,7 +109,13 @@ bool staged_wanted(const void *dev, const void *host) {
 hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device) {
     hipStream_t stream = ctx().stream;
     std::unique_lock<std::mutex> hold(g_stage.lock);
-    if (hipError_t e = stage_ready(); e != hipSuccess) return e;
+    if (stage_ready() != hipSuccess) {   // no pinned memory to be had: the runtime's own copy
+        (void)hipGetLastError();
+        hold.unlock();
+        const hipError_t e = to_device ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream)
+                                       : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);
+        return e != hipSuccess ? e : hipStreamSynchronize(stream);
+    }
     const int64_t n = (int64_t)((bytes + kStagePiece - 1) / kStagePiece);
     char *const h = (char *)host, *const d = (char *)dev;
     auto slot = [&](int64_t i) { return g_stage.ring + (i % kStageSlots) * kStagePiece; };
