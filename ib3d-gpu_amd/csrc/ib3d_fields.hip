@@ -592,6 +592,10 @@ k_momentum_lds(const double *__restrict__ u, const double *__restrict__ v, const
     // list what was skipped, one addition to the count per workgroup; the next
     // call's count is cleared here
     __shared__ int count[kMomTY], first;
+    // lane 0's mask for the whole wave: lanes past the last column have none of
+    // their own, but each lane lists the plane of its number
+    skipped = (uint64_t)(uint32_t)uniform((int)(uint32_t)(skipped >> 32)) << 32 |
+              (uint32_t)uniform((int)(uint32_t)skipped);
     if (tx == 0) count[ty] = __popcll(skipped);
     __syncthreads();
     int before = 0, all = 0;

@@ -13,7 +13,8 @@ OUT = ("ut", "vt", "wt", "resi_u", "resi_v", "resi_w")
 
 # cells per unit length of the uniform box, and the interior grid
 GRIDS = [(4, (66, 23, 17)), (4, (67, 24, 18)), (4, (68, 25, 19)), (8, (130, 33, 30)), (8, (131, 34, 31)),
-         (4, (33, 16, 38)), (10, (49, 66, 98))]
+         (4, (33, 16, 38)), (10, (49, 66, 98)),
+         (10, (69, 98, 98))]   # the last tile has 2 columns, a workgroup 6 planes
 
 
 def _fields(n, rng, odd):
