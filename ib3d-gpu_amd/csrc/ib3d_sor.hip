@@ -1738,38 +1738,44 @@ static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *is
     int64_t cap = 0, step = std::max(1, c.batch);
     for (; cap <= c.max_sweeps && step < 256; step = std::min<int64_t>(step * 2, 256)) cap += step;
     if (cap <= c.max_sweeps) cap += ((c.max_sweeps - cap) / step + 1) * step;
+    const int64_t most = cap / 2;   // launches up to it (the batches are even)
+    auto into_pc = [&](int from) {  // the values of buffer `from`
+        for (int col = 0; from && col < 2; col++)
+            IB3D_CHECK(hipMemcpyAsync(c.pc[col], g_pc2 + col * c.NC, c.NC * sizeof(double), hipMemcpyDeviceToDevice,
+                                      c.stream));
+        return 0;
+    };
     int64_t queued = 0, seen = 0;   // launches
     int size[2] = {0, 0};
     const double *prev = nullptr;
     for (int batch = 0;; batch++) {
         const int reg = batch & 1;
         const int64_t left = c.last_ref / 2 - queued;
-        const int n = left >= 96 ? kTrackBatch : left >= 48 ? 32 : 16;
-        double *region = g_track + reg * kRegion;
-        IB3D_CHECK(hipMemsetAsync(region, 0, n * kTrackSlots * sizeof(double), c.stream));
-        for (int q = 0; q < n; q++) {
-            double *slot = region + q * kTrackSlots;
-            launch64(c, P, 2, (int)((queued + q) & 1), omega, nullptr, epsi, prev, slot);
-            prev = slot;
+        const int n = (int)std::min<int64_t>(left >= 96 ? kTrackBatch : left >= 48 ? 32 : 16, most - queued);
+        if (n > 0) {
+            double *region = g_track + reg * kRegion;
+            IB3D_CHECK(hipMemsetAsync(region, 0, n * kTrackSlots * sizeof(double), c.stream));
+            for (int q = 0; q < n; q++) {
+                double *slot = region + q * kTrackSlots;
+                launch64(c, P, 2, (int)((queued + q) & 1), omega, nullptr, epsi, prev, slot);
+                prev = slot;
+            }
+            IB3D_CHECK(hipGetLastError());
+            IB3D_CHECK(hipMemcpyAsync(g_mirror + reg * kRegion, region, n * kTrackSlots * sizeof(double),
+                                      hipMemcpyDeviceToHost, c.stream));
+            IB3D_CHECK(hipEventRecord(g_batch_ev[reg], c.stream));
         }
-        IB3D_CHECK(hipGetLastError());
-        IB3D_CHECK(hipMemcpyAsync(g_mirror + reg * kRegion, region, n * kTrackSlots * sizeof(double),
-                                  hipMemcpyDeviceToHost, c.stream));
-        IB3D_CHECK(hipEventRecord(g_batch_ev[reg], c.stream));
         queued += n;
         size[reg] = n;
         if (batch == 0) continue;
         const int old = 1 - reg;
+        if (size[old] == 0) break;   // every launch up to the cap has been read
         IB3D_CHECK(hipEventSynchronize(g_batch_ev[old]));
         for (int q = 0; q < size[old]; q++, seen++) {
             for (int w = 0; w < 2; w++) {
                 const double *h = g_mirror + old * kRegion + q * kTrackSlots + w * kBlockSub;
                 double v = *std::max_element(h, h + kBlockSub);
                 const int64_t it = 2 * seen + w + 1;
-                if (it > cap) {
-                    set_error("REDBLACKSOR: no convergence within the sweep cap");
-                    return -1;
-                }
                 if (v >= epsi) continue;  // the reference loops while derr2 >= epsi
                 const int from = (int)(seen & 1);
                 int at = 1 - from;   // the buffer that holds the result
@@ -1784,10 +1790,7 @@ static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *is
                 } else if (w == 0) {
                     launch64(c, P, 1, from, omega, nullptr, 0.0);
                 }
-                if (at)
-                    for (int col = 0; col < 2; col++)
-                        IB3D_CHECK(hipMemcpyAsync(c.pc[col], g_pc2 + col * c.NC, c.NC * sizeof(double),
-                                                  hipMemcpyDeviceToDevice, c.stream));
+                if (into_pc(at)) return -1;
                 IB3D_CHECK(hipGetLastError());
                 *isum = it;
                 *derr2 = v;
@@ -1796,6 +1799,10 @@ static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *is
             }
         }
     }
+    // pc holds sweep `cap`, as the plain loop leaves it
+    if (into_pc((int)(most & 1))) return -1;
+    set_error("REDBLACKSOR: no convergence within the sweep cap");
+    return -1;
 }
 
 // subPcorVcor.f90:148-212 with the reference stopping rule.  Iterations are
