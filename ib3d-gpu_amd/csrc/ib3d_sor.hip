@@ -2683,6 +2683,7 @@ static SorGeom level_geom(const MgLevel &L) {
 }
 
 void mg_release() {
+    cycle_graph_release();   // (its launches hold the levels' buffers, x2 among them, which its key does not list)
     for (MgLevel &L : g_mg) {
         if (L.owns_tables) { (void)hipFree(L.ax); (void)hipFree(L.ay); (void)hipFree(L.az); }
         if (L.owns_xb) { (void)hipFree(L.x); (void)hipFree(L.b); }
