@@ -70,18 +70,26 @@ static_assert(kRecC + 12 <= kMomRec, "momentum record overflow");
 //   kChecked  numerators outside [2^-900, 2^900] (zeros, NaN and infinities
 //             among them) use the division instruction, so no intermediate
 //             leaves the normal range and signed zeros come out as from a / b
+//   kCheckedAlone  the same, its steps not shared with the forms below: the
+//             compiler then fits k_momentum_rows into 96 registers (with kChecked it
+//             spills 56 bytes, 798 us at 256x192x192 instead of 652); k_momentum is
+//             10% slower with it
 //   kPlain    the caller knows that a is zero or in that range and b > 0
 //   kPlainNeg the same, b < 0
 // The remainder of a zero is +0 and its quotient's sign that of a*y: the
 // correction adds -(b*q - a) * y for b > 0 and (a - b*q) * y for b < 0, both -0
 // there, so the zero keeps its sign.
-enum Quot { kDivide, kChecked, kPlain, kPlainNeg };
+enum Quot { kDivide, kChecked, kCheckedAlone, kPlain, kPlainNeg };
 template <Quot Q>
 __device__ __forceinline__ double dv(double a, double b, double y) {
     if (Q == kDivide) return a / b;
-    if (Q == kChecked) {
+    if (Q == kChecked || Q == kCheckedAlone) {
         const double m = fabs(a);
         if (!(m >= 0x1p-900 && m <= 0x1p900)) return a / b;
+        if (Q == kCheckedAlone) {
+            const double q = fma(fma(-b, a * y, a), y, a * y);
+            return fma(fma(-b, q, a), y, q);
+        }
     }
     double q = a * y;
     if (Q == kPlain) {
@@ -139,6 +147,26 @@ struct GlobalFields {
     template <int a, int b, int d> __device__ __forceinline__ double W() const { return w[c + a + b * sx + d * sxy]; }
     template <int a, int b, int d, class T> __device__ __forceinline__ T &at(T *base) const {
         return base[c + a + b * sx + d * sxy];
+    }
+    __device__ __forceinline__ void split() const {}
+};
+
+// GlobalFields32: the same values through 32-bit byte offsets from the uniform
+// array bases, one offset register per address instead of a 64-bit pair (fewer
+// registers, one more wave per SIMD).  For grids whose FP64 fields span less than
+// 4 GiB.
+struct GlobalFields32 {
+    const double *__restrict__ u, *__restrict__ v, *__restrict__ w;
+    uint32_t c, sx, sxy;  // element offsets; c * 8 < 2^32
+    template <int a, int b, int d, int S> __device__ __forceinline__ uint32_t off() const {
+        return (c + (uint32_t)a + (uint32_t)b * sx + (uint32_t)d * sxy) * (uint32_t)S;
+    }
+    template <int a, int b, int d> __device__ __forceinline__ double U() const { return at<a, b, d>(u); }
+    template <int a, int b, int d> __device__ __forceinline__ double V() const { return at<a, b, d>(v); }
+    template <int a, int b, int d> __device__ __forceinline__ double W() const { return at<a, b, d>(w); }
+    template <int a, int b, int d, class T> __device__ __forceinline__ T &at(T *base) const {
+        typedef std::conditional_t<std::is_const_v<T>, const char, char> B;
+        return *reinterpret_cast<T *>(reinterpret_cast<B *>(base) + off<a, b, d, (int)sizeof(T)>());
     }
     __device__ __forceinline__ void split() const {}
 };
@@ -369,7 +397,7 @@ __device__ __forceinline__ void momentum_cell(
 // k_momentum_lds has listed there.  The first `edge` workgroups take the wall
 // columns i = 2, nx, nx+1 of every row, kept out of the interior waves so that
 // those run one stencil branch.
-static constexpr int kRestBlocks = 1024;   // for the listed rows: as many waves as run at once
+static constexpr int kRestBlocks = 1024;   // for the listed rows (3072 of its 4096 waves run at once)
 template <bool FAST>
 __global__ void __launch_bounds__(256)
 k_momentum(const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w,
@@ -399,6 +427,28 @@ k_momentum(const double *__restrict__ u, const double *__restrict__ v, const dou
         const int i = r % tiles * 64 + lane + 3;
         if (i <= nx - 1) compute(i, r / tiles % ny + 2, r / tiles / ny + 2);
     }
+}
+
+// The interior columns of a large grid, one wave per row, on their own: with the
+// code for the wall columns beside them (k_momentum) the kernel needs 166 registers,
+// three waves per SIMD.  With 32-bit offsets and the fast divisions this fits 96,
+// five waves (the other forms need more and keep the compiler's choice).  A call
+// at 256x192x192 652 us, by k_momentum alone 707.
+template <bool FAST, bool OFF32>
+__global__ void __launch_bounds__(256, (FAST && OFF32) ? 5 : 1)
+k_momentum_rows(const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w,
+                const double *__restrict__ p, const int8_t *__restrict__ cell, double *__restrict__ ut,
+                double *__restrict__ vt, double *__restrict__ wt, double *__restrict__ ru, double *__restrict__ rv,
+                double *__restrict__ rw, Tabs T, MomTabs M, int nx, int ny, int nz, double rev, double deltat) {
+    const int64_t sx = nx + 2, sxy = sx * (ny + 2);
+    const int i = (int)blockIdx.x * 64 + (int)threadIdx.x + 3;
+    const int j = __builtin_amdgcn_readfirstlane((int)(blockIdx.y * 4 + threadIdx.y)) + 2, k = (int)blockIdx.z + 2;
+    if (j > ny + 1 || i > nx - 1) return;
+    const int64_t c = (i - 1) + sx * (j - 1) + sxy * (k - 1);
+    using Index = std::conditional_t<OFF32, uint32_t, int64_t>;
+    const std::conditional_t<OFF32, GlobalFields32, GlobalFields> A{u, v, w, (Index)c, (Index)sx, (Index)sxy};
+    momentum_cell<FAST ? kCheckedAlone : kDivide, false>(A, columns(T, M, i), {}, i, j, k, p, cell, ut, vt, wt, ru, rv,
+                                                         rw, M, nx, ny, nz, rev, deltat);
 }
 
 // The same interior columns, a 64 x 8 tile of (i, j) marching through tz planes.
@@ -847,6 +897,11 @@ static int g_mom_lds = 0;
 // its synchronisation, direct / tiles, us: 128x96x64 78 / 84, 160x80x80 106 / 98,
 // 190x128x100 193 / 150, 256x192x192 754 / 433).
 static constexpr int64_t kMomTilesFrom = 1000000;
+// From this many cells on the interior rows straight from HBM pay for a launch of
+// their own, k_momentum_rows (in k_momentum / apart, us: 128x64x64 42 / 52,
+// 128x88x88 73 / 77, 128x96x96 82 / 87, 160x100x96 125 / 122, 190x128x100 164 / 156,
+// 256x192x192 707 / 652).
+static constexpr int64_t kMomRowsFrom = 1500000;
 int set_momentum_tiles(int on) {
     IB3D_REQUIRE(on >= 0 && on <= 4, "set_momentum_tiles: variant must be 0..4");
     g_mom_lds = on;
@@ -887,6 +942,8 @@ int ns_momentum(Ctx &c, double rev, double deltat) {
     const int tz = momentum_planes((int64_t)tnx * tny, nz);
     const bool use_tiles = nxi > 0 && c.mom_plain && g_mom_lds != 4 &&
                            (g_mom_lds || (int64_t)nx * ny * nz >= kMomTilesFrom);
+    const bool apart = nxi > 0 && !use_tiles && (int64_t)nx * ny * nz >= kMomRowsFrom;
+    const bool off32 = c.P * (int64_t)sizeof(double) < ((int64_t)1 << 32);
     auto launch = [&](auto fast) {
         constexpr bool F = decltype(fast)::value;
         const int turn = c.mom_turn;
@@ -896,9 +953,13 @@ int ns_momentum(Ctx &c, double rev, double deltat) {
                                c.stream, c.u, c.v, c.w, c.p, c.tag, c.ut, c.vt, c.wt, c.resi_u, c.resi_v, c.resi_w,
                                c.mom_left + 2, c.mom_left + turn, c.mom_left + 1 - turn, T, M, nx, ny, nz, tz, rev, deltat);
         }
-        const int64_t rows = (int64_t)tnx * ny * nz;
+        if (apart)
+            hipLaunchKernelGGL((off32 ? k_momentum_rows<F, true> : k_momentum_rows<F, false>),
+                               dim3(tnx, nblocks(ny, 4), (unsigned)nz), dim3(64, 4, 1), 0, c.stream, c.u, c.v, c.w, c.p,
+                               c.tag, c.ut, c.vt, c.wt, c.resi_u, c.resi_v, c.resi_w, T, M, nx, ny, nz, rev, deltat);
+        const int rows = apart ? 0 : (int)((int64_t)tnx * ny * nz), row_blocks = (rows + 3) / 4;
         const int edge = nblocks((int64_t)3 * ny * nz, 256);
-        hipLaunchKernelGGL(k_momentum<F>, dim3(edge + (use_tiles ? std::min<int>(kRestBlocks, nblocks(rows, 4)) : (int)nblocks(rows, 4))),
+        hipLaunchKernelGGL(k_momentum<F>, dim3(edge + (use_tiles ? std::min(kRestBlocks, row_blocks) : row_blocks)),
                            dim3(256), 0, c.stream, c.u, c.v, c.w, c.p, c.tag, c.ut, c.vt, c.wt, c.resi_u, c.resi_v,
                            c.resi_w, use_tiles ? c.mom_left + 2 : nullptr, c.mom_left + turn, T, M, nx, ny, nz, edge, (int)tnx, rev, deltat);
     };
