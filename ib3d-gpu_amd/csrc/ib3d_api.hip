@@ -8,7 +8,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 
 #include "../../include/ib3d.h"
@@ -146,7 +145,7 @@ hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device) {
     int made = 0;
     try {
         for (; made < want; made++) pool[made] = std::thread(work, made, want);
-    } catch (const std::system_error &) {
+    } catch (...) {   // no thread, or no memory for one
     }
     hipError_t err = hipSuccess;
     if (made == want) {
@@ -158,12 +157,11 @@ hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device) {
                 void *const dp = d + (size_t)issued * kStagePiece, *const hp = slot(issued);
                 void *const to = to_device ? dp : hp, *const from = to_device ? hp : dp;
                 const int64_t len = (int64_t)size(issued);
-                const dim3 grid(kStageBlocks);
-                if (((uintptr_t)dev & 15) == 0)
-                    hipLaunchKernelGGL(k_stage<uint4>, grid, dim3(256), 0, stream, (uint4 *)to, (const uint4 *)from, len);
-                else
-                    hipLaunchKernelGGL(k_stage<uint2>, grid, dim3(256), 0, stream, (uint2 *)to, (const uint2 *)from, len);
-                err = hipGetLastError();
+                // (the launch's own status: hipGetLastError would also return an
+                // error that an earlier call of the user's program left behind)
+                const void *args[] = {&to, &from, &len};
+                err = hipLaunchKernel(((uintptr_t)dev & 15) == 0 ? (const void *)k_stage<uint4> : (const void *)k_stage<uint2>,
+                                      dim3(kStageBlocks), dim3(256), const_cast<void **>(args), 0, stream);
                 if (err == hipSuccess) err = hipEventRecord(g_stage.ev[q], stream);
                 issued++;
             } else if (synced < issued && (!to_device || issued == n || issued - synced >= kStageSlots / 2)) {
