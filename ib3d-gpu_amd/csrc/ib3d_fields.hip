@@ -881,8 +881,7 @@ static int build_mom_tables(Ctx &c) {
         c.mom_left = nullptr;
         c.mom_rows = 0;
         IB3D_CHECK(hipMalloc((void **)&c.mom_left, (rows + 2) * sizeof(int)));
-        IB3D_CHECK(dzero(c.mom_left, 2 * sizeof(int)));
-        c.mom_turn = 0;
+        c.mom_counts = false;
         c.mom_rows = rows;
     }
     c.mom_fast = fast;
@@ -944,11 +943,16 @@ int ns_momentum(Ctx &c, double rev, double deltat) {
                            (g_mom_lds || (int64_t)nx * ny * nz >= kMomTilesFrom);
     const bool apart = nxi > 0 && !use_tiles && (int64_t)nx * ny * nz >= kMomRowsFrom;
     const bool off32 = c.P * (int64_t)sizeof(double) < ((int64_t)1 << 32);
+    if (use_tiles && !c.mom_counts) {
+        IB3D_CHECK(dzero(c.mom_left, 2 * sizeof(int)));
+        c.mom_turn = 0;
+    }
     auto launch = [&](auto fast) {
         constexpr bool F = decltype(fast)::value;
         const int turn = c.mom_turn;
         if (use_tiles) {
             c.mom_turn = 1 - turn;
+            c.mom_counts = false;   // until the launches are known to have gone out
             hipLaunchKernelGGL(k_momentum_lds, dim3(tnx, tny, (unsigned)nblocks(nz, tz)), dim3(kMomTX, kMomTY, 1), 0,
                                c.stream, c.u, c.v, c.w, c.p, c.tag, c.ut, c.vt, c.wt, c.resi_u, c.resi_v, c.resi_w,
                                c.mom_left + 2, c.mom_left + turn, c.mom_left + 1 - turn, T, M, nx, ny, nz, tz, rev, deltat);
@@ -968,6 +972,7 @@ int ns_momentum(Ctx &c, double rev, double deltat) {
     else
         launch(std::false_type{});
     IB3D_CHECK(hipGetLastError());
+    if (use_tiles) c.mom_counts = true;
     return 0;
 }
 

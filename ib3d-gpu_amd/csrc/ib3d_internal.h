@@ -92,6 +92,7 @@ struct Ctx {
     int *mom_left = nullptr;   // two counts, used in turn, and the rows that k_momentum_lds leaves to k_momentum
     int64_t mom_rows = 0;      // room for rows
     int mom_turn = 0;
+    bool mom_counts = false;   // the count of this turn is zero (each call clears the next one's)
     bool mom_ready = false, mom_fast = false, mom_plain = false;
     // GMRES-IR iterations replayed as a captured HIP graph (ib3d_set_graphs)
     bool use_graphs = false;
