@@ -39,13 +39,13 @@ the learned form's measurement beside it.  After the timed steps, the
 configuration's whole stated run (500 steps, t = 1.0) of the headline mode
 and of the learned form is timed on its own (`full_run`).
 
-Roofline: for mode 4 the finest multigrid level's FP32 red-black sweep in one
-launch (k_sweep2_pz; the solver does two per launch); algorithmic bytes per
-launch = 12 B per interior cell (old value and right-hand side read, new
-value written, both colours).  For the SOR modes it is the half-sweep:
-16 B (FP64) or 8 B (FP32) per interior cell per launch.  The average launch
-duration is measured with HIP events on the library's stream
-(ib3d_bench_sor).
+Roofline: two red-black sweeps of the finest grid in one launch, as the solver
+does them (k_sor_march or k_sor_block by size), FP32 for the modes that smooth
+or sweep in FP32; algorithmic bytes per launch = 12 B (FP32) or 24 B (FP64) per
+interior cell (old value and right-hand side read, new value written, both
+colours).  Beside it the plain half-sweeps: 8 B or 16 B per interior cell per
+launch.  The average launch duration is measured with HIP events on the
+library's stream (ib3d_bench_sor).
 
 CPU baseline: the reference's own Fortran (built from its sources with
 amdflang -O3, oracle/_ref) timed on this host, one thread, on a bounded
@@ -250,13 +250,13 @@ def train_guess(cfg_name, rec_steps, epochs, batch, lr, omega, tol, inner):
 
 
 def kernel_roofline(s, precision, omega, n_cells, sweeps=200):
-    """precision 64 / 32: the half-sweep (two launches per sweep, 16 / 8 B per
-    cell each); 33: the FP32 whole sweep in one launch (12 B per cell)."""
-    s.bench_sor(precision, 5, omega)  # warm the tables and caches
+    """precision 65 / 34: two sweeps in one launch (FP64 24, FP32 12 B per cell);
+    64 / 32: the half-sweep (two launches per sweep, 16 / 8 B per cell each)."""
+    s.bench_sor(precision, 6, omega)  # warm the tables and caches
     ms = s.bench_sor(precision, sweeps, omega)
-    if precision == 33:
-        launch_s = ms * 1e-3
-        bytes_per_launch = 12.0 * n_cells
+    if precision in (34, 65):
+        launch_s = 2.0 * ms * 1e-3
+        bytes_per_launch = (24.0 if precision == 65 else 12.0) * n_cells
     else:
         launch_s = 0.5 * ms * 1e-3         # red and black launches per sweep
         bytes_per_launch = 0.5 * (32.0 if precision == 64 else 16.0) * n_cells
@@ -464,7 +464,7 @@ def main():
             prec, nsw = a.profile_sor
             ms = s.bench_sor(prec, nsw, a.omega)
             nx, ny, nz = cfg.n
-            nbytes = (8 if prec == 64 else 4) * nx * ny * nz
+            nbytes = (8 if prec in (64, 65) else 4) * nx * ny * nz
             cms = s.probe_copy(nbytes)
             print(json.dumps({"precision": prec, "sweeps": nsw, "ms_per_sweep": ms, "copy_bytes": nbytes,
                               "copy_ms": cms}), flush=True)
@@ -491,12 +491,11 @@ def main():
         main_fields = {f: s.download(f) for f in ("u", "p")}
         log(f"[bench] {a.mode}: {main_res}")
         prec = 32 if a.mode.startswith("mixed") or a.mode == "gmres-sor" else 64
-        # the smoother's sweep: the finest level's whole FP32 sweep in mode 4,
-        # the half-sweep otherwise
-        rprec = 33 if a.mode.startswith("mixed") else prec
+        # the solver's own launches on the finest grid, and the half-sweeps
+        rprec = 34 if prec == 32 else 65
         roof = kernel_roofline(s, rprec, a.omega, n_cells)
-        roof32 = kernel_roofline(s, 32, a.omega, n_cells) if rprec != 32 and prec == 32 else None
-        roof64 = kernel_roofline(s, 64, a.omega, n_cells) if prec == 32 else roof
+        roof32 = kernel_roofline(s, 32, a.omega, n_cells) if prec == 32 else None
+        roof64 = kernel_roofline(s, 64, a.omega, n_cells)
         s.close()
         if "mixed+learned" in modes and net is None:
             tt = time.perf_counter()
@@ -531,11 +530,11 @@ def main():
         if os.path.exists(tf):
             with open(tf) as fh:
                 t = json.load(fh)
-            traffic = t.get({33: "fp32_sweep", 32: "fp32", 64: "fp64"}[rprec])
+            traffic = t.get({34: "fp32_pair", 65: "fp64_pair"}[rprec])
         roof_out = {k: roof[k] for k in ("bound", "achieved", "peak", "unit", "frac")}
         roof_out["traffic"] = traffic
-        roof_out["kernel"] = ("k_sweep2_pz: FP32 red-black sweep in one launch (12 B per cell)" if rprec == 33 else
-                              f"k_sor_pz<{'float' if prec == 32 else 'double'}> half-sweep")
+        roof_out["kernel"] = (f"k_sor_march or k_sor_block<{'float' if prec == 32 else 'double'}>: two red-black sweeps "
+                              f"in one launch ({12 if prec == 32 else 24} B per cell)")
         roof_out["launch_us"] = roof["launch_us"]
         # what a plain streaming copy reaches on this device (604 MB read and
         # written), for reading `frac` against a practical ceiling

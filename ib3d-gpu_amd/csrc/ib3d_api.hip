@@ -1218,8 +1218,9 @@ int ib3d_step(int first, double rev, double re, double deltat, double eps1, doub
 int ib3d_bench_sor(int precision, int sweeps, double omega, double *ms_per_sweep) {
     Ctx &c = ctx();
     IB3D_REQUIRE(c.ready && c.matrix_ready, "bench_sor: setup incomplete");
-    IB3D_REQUIRE(precision == 64 || precision == 32 || precision == 33,
-                 "bench_sor: precision must be 64, 32 or 33 (FP32, one launch per sweep)");
+    IB3D_REQUIRE(precision == 64 || precision == 65 || (precision >= 32 && precision <= 34),
+                 "bench_sor: precision must be 64 or 32 (half-sweep launches), 33 (FP32, one launch per sweep), 65 or 34 "
+                 "(FP64, FP32, two sweeps per launch)");
     IB3D_REQUIRE(sweeps >= 1, "bench_sor: sweeps must be >= 1");
     return bench_sor(c, precision, sweeps, omega, ms_per_sweep);
 }

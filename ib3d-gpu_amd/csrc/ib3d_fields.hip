@@ -463,12 +463,12 @@ k_momentum_rows(const double *__restrict__ u, const double *__restrict__ v, cons
 // host has found the tables fit for it).  The others are listed in `left` for
 // k_momentum.  With the general cell in this kernel the compiler spilled.
 //
-// Bounded by FP64 issue (518 of 680 vector instructions per row; 211 us at 256 x
-// 192 x 192) and latency at four waves per SIMD: 338 us there, 1.75 ms at
-// 512 x 320 x 320 (3.55 before), and 66 and 405 us for the rows it leaves.  Reading every stencil value and table through the vector
-// cache, 107 eight-byte loads per row that it serves at 16 clocks each, took
-// 640 us; the tiles with a tested quotient each, and the general cell beside it,
-// 410.
+// Bounded by FP64 issue (486 of 692 vector instructions per row; 220 us of issue at
+// 256 x 192 x 192) and latency at four waves per SIMD: 338 us there, 1.75 ms at
+// 512 x 320 x 320 (3.55 before), and 66 and 405 us for the rows it leaves.  Reading
+// every stencil value and table through the vector cache, 108 eight-byte loads per
+// row that it serves at 16 clocks each, took 640 us; the tiles with a tested quotient
+// each, and the general cell beside it, 410.
 __global__ void __launch_bounds__(kMomTX * kMomTY, 4)
 k_momentum_lds(const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w,
                const double *__restrict__ p, const int8_t *__restrict__ cell, double *__restrict__ ut,

@@ -1537,8 +1537,8 @@ static int second_e(Ctx &c) {
 // 24x16x8 | march:
 //   18k cells  14.9 |  3.5 |  4.3 |  6.5 |           49k  17.6 |  4.1 |  4.4 |  6.5 |
 //   147k       17.8 |  6.3 |  6.0 |  6.9 |           301k 18.7 | 10.0 |  7.7 |  7.5 |
-//   524k       16.5 | 14.9 | 11.2 |  8.2 | 11.4      1.47M 20.1 |     | 22.3 | 15.1 | 16.8
-//   1.70M      21.3 |      | 27.5 | 20.9 | 17.9      9.4M  66.8 |     |      |      | 35.4
+//   524k       16.5 | 14.9 | 11.2 |  8.2 | 11.4      1.47M 20.1 |     | 22.3 | 15.1 | 12.7
+//   1.70M      21.3 |      | 27.5 | 20.9 | 13.7      9.4M  66.8 |     |      |      | 35.4
 //   25M       180.0 |      |      |      | 87.2
 // and per FP32 sweep, half-sweep launches | 8x8x4 | 24x8x8 | march:
 //   18k  11.7 | 2.6 |  3.1 |        66k  16.1 | 2.8 |  3.2 |  5.0     147k 14.9 | 3.6 | 3.4 | 5.1
@@ -2912,7 +2912,7 @@ static dim3 level_grid(const MgLevel &L) {
 static int g_fused = 2;          // levels (from the finest) smoothed by whole sweeps in one launch
 static int g_coarse_tiles = 2;   // first level smoothed by two temporally blocked launches per phase (0: none)
 static int g_fused_restrict = 64;  // levels (from the finest) whose residual is restricted in one pass
-static int g_prolong_pz = 2;       // levels (from the finest) prolonged four cells of a row per thread
+static int g_prolong_pz = 2;       // levels (from the finest) prolonged by 4 x 2 x 2 cells per thread
 static int g_sweep_tz = 0;        // planes per chunk on the finest level (0: from g_sweep_blocks)
 static constexpr int kSweepBlocks = 480, kSweepBlocksCoarse = 192;
 static int g_sweep_blocks = kSweepBlocks;
@@ -3533,7 +3533,7 @@ int bench_sor(Ctx &c, int precision, int sweeps, double omega, double *ms) {
     hipEvent_t a, b;
     IB3D_CHECK(hipEventCreate(&a));
     IB3D_CHECK(hipEventCreate(&b));
-    if (precision == 32 || precision == 33) {
+    if (precision < 64) {
         if (sor_float_tables(c)) return -1;
         const unsigned nb = nblocks(2 * c.NC, kSorBlock);
         if (ensure_partial(nb)) return -1;
@@ -3541,8 +3541,9 @@ int bench_sor(Ctx &c, int precision, int sweeps, double omega, double *ms) {
                            c.e32[1], c.bdt[0], c.bdt[1], c.r32[0], c.r32[1], c.ax, c.ay, c.az, geom(c), c.partial,
                            nullptr, 0.0);
     }
-    // 33: the fused FP32 sweep (one launch per red-black sweep) between e32
-    // and a second buffer, as on the finest multigrid level
+    // 34, 65: two sweeps per launch as the solver plans them for this grid, between
+    // the unknown (e32, pc) and its second buffer.  33: k_sweep2_pz, one sweep per
+    // launch, between the same buffers as 34.
     // After a mode-4 solve it sweeps the solver's own buffers (the first
     // Krylov vector z from the first basis vector v, and the multigrid's
     // second buffer), so the probe reads and writes the memory the solver's
@@ -3554,10 +3555,18 @@ int bench_sor(Ctx &c, int precision, int sweeps, double omega, double *ms) {
     bool own_x2 = false;
     int S = 0, tz = 0;
     dim3 sg;
-    if (precision == 33) {
-        if (sor_float_tables(c)) return -1;
-        L.sx = c.sx; L.sy = c.sy; L.sz = c.sz; L.H = c.H; L.NC = c.NC; L.sxp = c.sxp;
-        IB3D_REQUIRE(sweep2_shape(L, S, tz, sg), "bench_sor: the fused sweep does not fit this grid");
+    SweepPlan P;
+    const bool pairs = precision == 34 || precision == 65;
+    if (pairs) {
+        P = precision == 34 ? plan32(c) : plan64(c);
+        IB3D_REQUIRE(P.kind, "bench_sor: this grid is not swept two at a time");
+        if (precision == 65 && second_pc(c)) return -1;
+    }
+    if (precision == 33 || precision == 34) {
+        if (precision == 33) {
+            L.sx = c.sx; L.sy = c.sy; L.sz = c.sz; L.H = c.H; L.NC = c.NC; L.sxp = c.sxp;
+            IB3D_REQUIRE(sweep2_shape(L, S, tz, sg), "bench_sor: the fused sweep does not fit this grid");
+        }
         if (!g_mg.empty() && g_mg[0].x2 && g_mg[0].NC == c.NC) {
             x2 = g_mg[0].x2;
             if (g_kv && g_kz && g_k_nc == c.NC) {
@@ -3574,9 +3583,15 @@ int bench_sor(Ctx &c, int precision, int sweeps, double omega, double *ms) {
     const SorGeom g = geom(c);
     const float om = (float)omega, omm = (float)(1.0 - omega);
     float *xa = x0, *xb = x2;
+    const int launches = pairs ? (sweeps + 1) / 2 : sweeps;
     IB3D_CHECK(hipEventRecord(a, c.stream));
-    for (int q = 0; q < sweeps; q++) {
-        if (precision == 33) {
+    for (int q = 0; q < launches; q++) {
+        if (precision == 34) {
+            launch32(c, P, 2, xa, xb, rhs0, omega, false, nullptr);
+            std::swap(xa, xb);
+        } else if (precision == 65) {
+            launch64(c, P, 2, q & 1, omega, nullptr, 0.0);
+        } else if (precision == 33) {
             hipLaunchKernelGGL(k_sweep2_pz<false>, sg, dim3(kSweepThreads), 0, c.stream, xa, xa + c.NC, xb,
                                xb + c.NC, rhs0, rhs1, g_axf, g_ayf, g_azf, g, S, tz, om, omm, nullptr, 0.0);
             std::swap(xa, xb);
@@ -3590,7 +3605,7 @@ int bench_sor(Ctx &c, int precision, int sweeps, double omega, double *ms) {
     IB3D_CHECK(hipEventSynchronize(b));
     float t = 0;
     IB3D_CHECK(hipEventElapsedTime(&t, a, b));
-    *ms = (double)t / sweeps;
+    *ms = (double)t / (pairs ? 2 * launches : sweeps);
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     if (x2) {

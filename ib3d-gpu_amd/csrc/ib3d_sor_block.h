@@ -35,8 +35,7 @@
 // which walks eight planes through two dependent loads (7-9 us whatever the
 // grid).  us per FP64 sweep with TRACK, k_sor_pz -> here: 14.9 -> 3.5 at
 // 32x24x24, 17.6 -> 4.1 at 48x32x32, 17.8 -> 6.0 at 64x48x48, 16.5 -> 8.2 at
-// 128x64x64, 20.1 -> 15.1 at 160x96x96; FP32: 14.4 -> 3.1 at 48x32x32, 14.8 ->
-// 3.3, 12.7 -> 4.8, 15.5 -> 8.3.
+// 128x64x64; FP32: 14.4 -> 3.1 at 48x32x32, 14.8 -> 3.3, 12.7 -> 4.8.
 //
 // Measured and dropped: one sweep per launch (28 x 12 x 8 blocks: 9.1 us at
 // 128x64x64, 7.2 at 48x32x32), three (6.1 at 48x32x32), columns of both
@@ -60,7 +59,7 @@ static constexpr int kBlockSub = 16;
 template <int M, int OX, int OY, int OZ> struct BlockShape {
     static constexpr int R = 2 * M, EX = OX + 2 * R, EY = OY + 2 * R, EZ = OZ + 2 * R;
     static constexpr int HX = EX / 2, HALF = HX * EY, HP = (HALF + 63) / 64 * 64, NT = 2 * HP, N2 = EZ / 2;
-    static_assert(2 * N2 <= 32 && OX % 2 == 0 && OZ % 2 == 0 && NT <= 1024, "block shape");
+    static_assert(M <= 2 && 2 * N2 <= 32 && OX % 2 == 0 && OZ % 2 == 0 && NT <= 1024, "block shape");
 };
 
 // a / b in two parts: the reciprocal, once per cell and launch, and the
@@ -260,10 +259,6 @@ k_sor_block(const T *__restrict__ s0, const T *__restrict__ s1, T *__restrict__ 
     if constexpr (M >= 2) {
         sweep_half(std::integral_constant<int, 3>{});
         sweep_half(std::integral_constant<int, 4>{});
-    }
-    if constexpr (M >= 3) {
-        sweep_half(std::integral_constant<int, 5>{});
-        sweep_half(std::integral_constant<int, 6>{});
     }
     if (own) {
 #pragma unroll

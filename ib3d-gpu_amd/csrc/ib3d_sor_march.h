@@ -34,9 +34,9 @@
 // 160 updates per slot of a chunk of 32 planes (FP64 with TRACK 38.0 -> 35.4 us per
 // sweep at 256x192x192, FP32 17.3 -> 16.5).
 //
-// What bounds it: vector arithmetic (55-60% of the issue slots; the rest is the
-// four updates' chain, 15 LDS reads per step and the barrier, at four waves per
-// SIMD), of which the halo is 1.65 times at 256x192x192.  us per sweep, k_sor_pz
+// What bounds it: vector arithmetic (58% of the issue slots in FP32, 69% in FP64;
+// the rest is the four updates' chain, 15 LDS reads per step and the barrier, at four
+// waves per SIMD), of which the halo is 1.65 times at 256x192x192.  us per sweep, k_sor_pz
 // (FP32: k_sweep2_pz) -> here: FP64 with TRACK 66.8 -> 35.4 at 256x192x192, 180 ->
 // 92 at 384x256x256 (the half-sweeps' atomicMax and, from 384x256x256 on, an
 // Infinity Cache that no longer holds the arrays); FP32 25-28 -> 16.5 at

@@ -219,9 +219,9 @@ int ib3d_set_fused_restrict(int levels);
  * test instead, which reads outside. */
 int ib3d_selfcheck_resid_guard(int64_t nx, int64_t ny, int64_t nz, int drop_interior, int64_t *outside);
 /* nsMomentum's interior columns: on == 0 (the default) chooses by size; 1, 2,
- * 3 march LDS tiles of 64 x 8 columns in z, with the rows that need a branch in
- * a second launch; 4 reads every stencil value from HBM.  All give identical
- * results. */
+ * 3 (three names for one form) march LDS tiles of 64 x 8 columns in z, with the
+ * rows that need a branch in a second launch; 4 reads every stencil value from
+ * HBM.  All give identical results. */
 int ib3d_set_momentum_tiles(int on);
 /* modes 3 and 4: replay each refinement iteration (Krylov cycle, FP64
  * residual and its norm) as one captured HIP graph (on != 0) or launch its
@@ -246,9 +246,10 @@ int ib3d_residual_norm(double *rnorm, double *bnorm);
 int ib3d_step(int first, double rev, double re, double deltat, double eps1, double out[8]);
 
 /* Kernel micro-benchmark used for the roofline figure: `sweeps` RB-SOR
- * sweeps (precision 64 or 32: two half-sweep launches each; 33: FP32, one
- * launch per sweep, as on the finest multigrid level) on the current
- * right-hand side, timed with HIP events on the library stream.
+ * sweeps (precision 65 or 34: FP64 or FP32, two sweeps per launch, as the
+ * solver does them on this grid; 64 or 32: two half-sweep launches each; 33:
+ * FP32, one launch per sweep) on the current right-hand side, timed with HIP
+ * events on the library stream.
  * ms_per_sweep = average duration of one red+black sweep. */
 int ib3d_bench_sor(int precision, int sweeps, double omega, double *ms_per_sweep);
 /* Diagnostics (no reference counterpart): one streaming device copy of
