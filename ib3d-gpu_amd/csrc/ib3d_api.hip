@@ -4,6 +4,7 @@
 
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -52,10 +53,14 @@ void ib_release();
 // kernel moves each between the ring and the device (the copy engine needs 15 us
 // more per piece): 1.86 ms down (42 GB/s) and 1.97 up.  Eight threads are no
 // faster than four, pieces of 512 KB reach 36 GB/s, of 2 MB 44 for twice the
-// ring.  The calling thread alone makes HIP calls, so the workers need no device
-// of their own; they end before the call returns.
+// ring.  A thread that has nothing to do for some 20 us sleeps: where other processes
+// keep all CPUs busy, threads that yield instead hand over whole time slices (78 MB
+// up 64 ms, down 36; sleeping 7.5 and 11.4, the runtime 6.7 and 15.4).  The calling
+// thread alone makes HIP calls, so the workers need no device of their own; they
+// end before the call returns.
 static constexpr int kStageThreads = 4, kStageSlots = 16, kStageBlocks = 64;
 static constexpr size_t kStagePiece = size_t(1) << 20;
+static constexpr int kStageSpin = 500;
 struct Stage {
     std::mutex lock;              // one transfer at a time uses the ring
     char *ring = nullptr;         // kStageSlots pinned pieces
@@ -93,10 +98,19 @@ static hipError_t stage_ready() {
     return hipHostMalloc((void **)&g_stage.ring, kStageSlots * kStagePiece, hipHostMallocDefault);
 }
 
+// the CPUs this thread may run on
+static int host_cpus() {
+    cpu_set_t set;
+    return sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
+}
+
 // whether `host` is ordinary memory (a pinned or a device pointer is copied
-// directly) and the device's side is aligned for k_stage
-bool staged_wanted(const void *dev, const void *host) {
-    if (!host || ((uintptr_t)dev & 7)) return false;
+// directly), the device's side is aligned for k_stage, and there are CPUs for the
+// copy threads to gain on: one more than the calling thread's for a download
+// (78 MB 6.2 ms, by the runtime 7.9), two for an upload (2.3 and 2.7; with one
+// 2.9)
+bool staged_wanted(const void *dev, const void *host, bool to_device) {
+    if (!host || ((uintptr_t)dev & 7) || host_cpus() < (to_device ? 3 : 2)) return false;
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, host) != hipSuccess) {
         (void)hipGetLastError();
@@ -124,23 +138,36 @@ hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device) {
     std::atomic<int64_t> open{to_device ? (int64_t)kStageSlots : 0};
     std::atomic<int64_t> done[kStageSlots] = {};
     std::atomic<bool> stop{false};
+    std::mutex m;
+    std::condition_variable opened, moved;
+    auto tell = [&](std::condition_variable &cv) {
+        { std::lock_guard<std::mutex> l(m); }   // (a waiter has tested before, or sees the change)
+        cv.notify_all();
+    };
+    auto await = [&](std::condition_variable &cv, auto ready) {
+        for (int spin = 0; spin < kStageSpin; spin++) {
+            if (ready()) return;
+            __builtin_ia32_pause();
+        }
+        std::unique_lock<std::mutex> l(m);
+        cv.wait(l, ready);
+    };
     auto work = [&](int64_t first, int64_t stride) {
         for (int64_t i = first; i < n; i += stride) {
-            for (int spin = 0; open.load(std::memory_order_acquire) <= i; spin++) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                if (spin > 1000) std::this_thread::yield();
-            }
+            await(opened, [&] {
+                return open.load(std::memory_order_acquire) > i || stop.load(std::memory_order_acquire);
+            });
+            if (open.load(std::memory_order_acquire) <= i) return;
             char *mine = h + (size_t)i * kStagePiece;
             if (to_device)
                 std::memcpy(slot(i), mine, size(i));
             else
                 std::memcpy(mine, slot(i), size(i));
             done[i % kStageSlots].store(i + 1, std::memory_order_release);
+            tell(moved);
         }
     };
-    cpu_set_t set;
-    const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
-    const int want = (int)std::min<int64_t>(n, std::max(1, std::min(kStageThreads, cpus - 1)));
+    const int want = (int)std::min<int64_t>(n, std::max(1, std::min(kStageThreads, host_cpus() - 1)));
     std::thread pool[kStageThreads];
     int made = 0;
     try {
@@ -167,12 +194,19 @@ hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device) {
             } else if (synced < issued && (!to_device || issued == n || issued - synced >= kStageSlots / 2)) {
                 err = hipEventSynchronize(g_stage.ev[synced % kStageSlots]);
                 synced++;
-                if (err == hipSuccess)
+                if (err == hipSuccess) {
                     open.store(to_device ? synced + kStageSlots : synced, std::memory_order_release);
+                    tell(opened);
+                }
+            } else {
+                await(moved, [&] { return done[q].load(std::memory_order_acquire) != seen; });
             }
         }
     }
-    if (made < want || err != hipSuccess) stop.store(true);
+    if (made < want || err != hipSuccess) {
+        stop.store(true);
+        tell(opened);
+    }
     for (int t = 0; t < made; t++) pool[t].join();
     if (err != hipSuccess) {
         (void)hipStreamSynchronize(stream);   // (nothing may use the ring after the lock is given back)

@@ -276,17 +276,17 @@ void launch_max_partials(const double *partial, int64_t n, double *out);
 // costs as much), uploads from 32 MB on (14.5 MB 0.40 ms by the runtime, 0.45
 // staged; 78 MB 2.76 and 1.97).
 static constexpr size_t kStageDown = size_t(2) << 20, kStageUp = size_t(32) << 20;
-bool staged_wanted(const void *dev, const void *host);
+bool staged_wanted(const void *dev, const void *host, bool to_device);
 hipError_t staged_copy(void *dev, void *host, size_t bytes, bool to_device);
 inline hipError_t h2d(void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return hipSuccess;
-    if (bytes >= kStageUp && staged_wanted(dst, src)) return staged_copy(dst, const_cast<void *>(src), bytes, true);
+    if (bytes >= kStageUp && staged_wanted(dst, src, true)) return staged_copy(dst, const_cast<void *>(src), bytes, true);
     hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx().stream);
     return e != hipSuccess ? e : hipStreamSynchronize(ctx().stream);
 }
 inline hipError_t d2h(void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return hipSuccess;
-    if (bytes >= kStageDown && staged_wanted(src, dst)) return staged_copy(const_cast<void *>(src), dst, bytes, false);
+    if (bytes >= kStageDown && staged_wanted(src, dst, false)) return staged_copy(const_cast<void *>(src), dst, bytes, false);
     hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx().stream);
     return e != hipSuccess ? e : hipStreamSynchronize(ctx().stream);
 }
