@@ -1,0 +1,71 @@
+"""Solves of changing length.  A solve queues its sweeps in batches sized by the
+previous solve's count: short after long, long after short and one after the other
+the counts and every value of pc must be the oracle's, under the reference rule and
+in the FP64 L2 mode (whose FP32 form sweeps and counts by the same loop), and a solve
+that ends at once must not wait for what a long one would have needed (batches of
+1023 outer iterations: 40 times as long; medians of five, bound by a factor of ten)."""
+import time
+
+import numpy as np
+import pytest
+from test_gpu_sor_blocks import _pair, _same
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(4, (33, 25, 23)), (8, (65, 63, 64)), (12, (119, 93, 73))]
+
+
+@pytest.mark.parametrize("per,n", GRIDS)
+def test_counts_match_the_oracle(tmp_path, per, n):
+    s, o = _pair(tmp_path, per, n)
+    try:
+        s.computeDiv()
+        o.compute_div()
+        for eps in (0.3, 1e300, 0.3, 1e300, 1e300, 0.5, 0.2):
+            if eps < 1e300:
+                for a in ("pc", "pco"):
+                    o.array(a)[:] = 0.0
+                s.upload("pc", o.array("pc"))
+            it, d2 = s.REDBLACKSOR(eps)
+            print(f"[gpu] solve lengths {n} eps={eps}: {it} sweeps", flush=True)
+            assert (it, d2) == o.redblack_sor(eps)
+            assert _same(s.download("pc"), o.array("pc"))
+        fields = {f: np.asfortranarray(o.field(f)) for f in ("ut", "vt", "wt")}
+        for check, tol in ((1, 0.5), (1, 0.02), (1, 0.9), (3, 0.02), (3, 0.9), (3, 0.1), (10, 0.01), (10, 0.9), (10, 0.01)):
+            for f, a in fields.items():   # (a solve corrects them)
+                s.upload(f, a)
+            s.set_poisson_mode(1, omega=1.7, tol=tol, check=check, warm=False)
+            s.poissonSolver()
+            o.array("pc")[:] = 0.0
+            it, rel = o.sor_l2(1.7, tol, 100000, check)
+            print(f"[gpu] solve lengths {n} check={check} tol={tol}: {it} sweeps", flush=True)
+            assert s.poisson_stats()["sweeps"] == it
+            assert _same(s.download("pc"), o.array("pc"))
+    finally:
+        s.close()
+
+
+def test_a_short_solve_after_a_long_one(tmp_path):
+    s, o = _pair(tmp_path, *GRIDS[0])
+    try:
+        fields = {f: np.asfortranarray(o.field(f)) for f in ("ut", "vt", "wt")}
+
+        def solve(tol):
+            for f, a in fields.items():
+                s.upload(f, a)
+            s.set_poisson_mode(1, omega=1.0, tol=tol, check=1, warm=False)
+            s.sync()
+            t = time.perf_counter()
+            s.poissonSolver()
+            return time.perf_counter() - t, s.poisson_stats()["sweeps"]
+        for _ in range(2):
+            solve(0.9)
+        alone = sorted(solve(0.9)[0] for _ in range(5))[2]
+        after = []
+        for _ in range(5):
+            assert solve(1e-6)[1] > 1100
+            after.append(solve(0.9)[0])
+        print(f"[gpu] a short solve: {1e3 * alone:.2f} ms, after a long one {1e3 * sorted(after)[2]:.2f} ms", flush=True)
+        assert sorted(after)[2] < 10.0 * alone
+    finally:
+        s.close()
