@@ -1727,8 +1727,8 @@ static void launch32(Ctx &c, const SweepPlan &P, int M, const float *src, float 
 // which a sweep falls below epsi stops those after it.  If that was its first
 // sweep the launch holds one too many, and the march records only whether a
 // value reached epsi: then the one or two sweeps are repeated from the launch's
-// source.  The first two batches are small, the next large until the previous
-// solve's count is near, small after: a launch queued after convergence still
+// source.  Batches are large until the previous solve's count is near, small
+// after, smallest where that count was: a launch queued after convergence still
 // costs about 3 us.
 static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *isum, double *derr2) {
     const double omega = 1.99;
@@ -1752,9 +1752,8 @@ static int reference_blocks(Ctx &c, const SweepPlan &P, double epsi, int64_t *is
     for (int batch = 0;; batch++) {
         const int reg = batch & 1;
         const int64_t left = c.last_ref / 2 - queued;
-        const int few = c.last_ref > 0 && c.last_ref <= 8 ? 4 : 8;
-        const int n = (int)std::min<int64_t>(batch < 2 ? few : left >= 96 ? kTrackBatch : left >= 48 ? 32 : 16,
-                                             most - queued);
+        const int few = batch < 2 && c.last_ref > 0 && c.last_ref <= 8 ? 4 : 16;
+        const int n = (int)std::min<int64_t>(left >= 96 ? kTrackBatch : left >= 48 ? 32 : few, most - queued);
         if (n > 0) {
             double *region = g_track + reg * kRegion;
             IB3D_CHECK(hipMemsetAsync(region, 0, n * kTrackSlots * sizeof(double), c.stream));
@@ -1935,13 +1934,13 @@ static int sor_l2(Ctx &c, bool mixed, double bn, int64_t *sweeps, int64_t *outer
     // Batches of outer iterations are queued one ahead of the batch the host
     // reads (through the pinned mirror), so the GPU never waits for the host.
     // The previous solve's count predicts this one's (warm starts, slowly
-    // varying flow): up to 32 at a time until a little less than that, then a
-    // few, since a launch queued after convergence still costs about 2 us (a
-    // solve of 7 iterations after one of 11298 waited 15 ms for what was queued
-    // at 1023 at a time).
+    // varying flow): up to 64 at a time (32 in the first two batches) until a
+    // little less than that, then a few, since a launch queued after convergence
+    // still costs about 2 us (a solve of 7 iterations after one of 11298 waited
+    // 15 ms for what was queued at 1023 at a time), and a batch about 10.
     auto ahead = [&](int batch) {
-        const int few = batch < 2 || o <= c.last_outer + 2 ? 2 : 4;
-        return (int)std::min<int64_t>(32, std::max<int64_t>(few, c.last_outer - 4 - o));
+        const int64_t few = c.last_outer < 16 ? 2 : 4;
+        return (int)std::min<int64_t>(batch < 2 ? 32 : 64, std::max(few, c.last_outer - 4 - o));
     };
     struct Batch { int64_t from, to; };
     Batch pending[2];
