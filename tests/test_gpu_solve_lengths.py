@@ -3,7 +3,7 @@ previous solve's count: short after long, long after short and one after the oth
 the counts and every value of pc must be the oracle's, under the reference rule and
 in the FP64 L2 mode (whose FP32 form sweeps and counts by the same loop), and a solve
 that ends at once must not wait for what a long one would have needed (batches of
-1023 outer iterations: 70 times as long as after a short one, of 32 five times;
+1023 outer iterations: 70 times as long as after a short one, of 32 up to ten;
 medians of five, bound by a factor of thirty)."""
 import time
 
